@@ -235,7 +235,7 @@ int finish_powspec(pk_plan* p, const Job& j, hipStream_t s, bool fused = false) 
   const int n = p->n;
   int e = fused ? fft_ypass_mass(n, j, p->tw, s) : fft_ypass(n, j, p->tw, s);
   if (e) return e;
-  const int G = bin_grid(n, j.nb);
+  const int G = bin_blocks(n, j.nb);
   e = fft_xpass_bin(n, j, p->tw, G, s);
   if (e) return e;
   return bin_finalize(j, G, s);

@@ -292,7 +292,7 @@ __device__ __forceinline__ int find_bin(int m, const int* __restrict__ thr, cons
   return b;
 }
 
-constexpr int HB_LDS = 256;   // bins held in LDS; above this the per-block slice lives in HBM
+constexpr int HB_LDS = 256;   // bins of the binning x pass's usual LDS histogram
 constexpr int NACC = BIN_PART_LEN;   // S0, S2, S4 and the binned mode count per block and bin
 
 // Exponent e of the bins' 64-bit fixed point (a sum is an integer times 2^-e).  Every entry
@@ -328,51 +328,81 @@ __device__ __forceinline__ unsigned long long to_bin_fixed(float v, double scale
 // Each persistent block accumulates its own histogram and writes it to
 // partials[block][nb][NACC] once at the end.
 // ------------------------------------------------------------------------------------
-// LDS of the binning x pass and the waves per SIMD it leaves room for; the register
-// budget is held to that so registers never cost a resident block
-template <int N> struct XBinLds {
-  static constexpr size_t TILE = (size_t)N * (FFTCfg<N>::CX + 1) * 8;
+// Where a block of the binning x pass keeps its histogram, by the number of bins:
+//   XB_LDS  up to HB_LDS bins, static LDS (not at N = 1024, where XB_TALL is faster);
+//   XB_TALL up to its capacity (N = 512 and 1024 only), dynamic LDS: one block of 1024
+//           threads per CU with a tile of twice the columns (32 at 512, 16 at 1024).  At 512 the
+//           histogram and two of the usual 16-column tiles do not fit 160 KB, and one alone
+//           would leave half the waves; at 1024 a 16-column tile fills its 128-byte lines and
+//           bins by quads (512 bins at 1024^3: 1549 us, against 2463 us for XB_WIDE);
+//   XB_WIDE up to its capacity, dynamic LDS beside the usual tile;
+//   XB_HBM  the block's slice of the partials in HBM (device atomics), beyond that.
+// Device atomics cost far more than any tile: 443 bins at 512^3 took 2305 us with them and
+// take 251 us in XB_TALL; 512 bins at 1024^3 took 15410 us.
+enum { XB_HBM = 0, XB_LDS = 1, XB_TALL = 2, XB_WIDE = 3 };
+constexpr size_t LDS_BYTES = 160 * 1024;
+
+// tile, LDS and the waves per SIMD it leaves room for; the register budget is held to that so
+// registers never cost a resident block
+template <int N, int M> struct XBin {
+  static constexpr bool TALL_OK = N == 512 || N == 1024;
+  static constexpr int C = (M == XB_TALL && TALL_OK) ? (N == 512 ? 32 : 16) : FFTCfg<N>::CX;
+  static constexpr int NT = (M == XB_TALL && TALL_OK) ? 1024 : FFTCfg<N>::NTX;
   static constexpr int JLEN = isqrt_c(3 * (N / 2) * (N / 2)) + 2;   // isqrt-start table entries
-  static constexpr size_t HIST =
-      (size_t)(HB_LDS + 1) * 4 + 3 * HB_LDS * 8 + HB_LDS * 4 + (size_t)(N / 2 + 1) * 4 + (size_t)JLEN * 2 +
-      (size_t)(N / 2) * 8;
-  // LDS-limited waves per SIMD (the histogram in HBM: no limit is imposed)
-  template <bool LH> static constexpr int wpe() {
-    return LH ? cmax(1, cmin(4, (int)((160 * 1024) / (TILE + HIST)) * (FFTCfg<N>::NTX / 64) / 4)) : 1;
+  static constexpr size_t TILE = (size_t)N * (C + 1) * 8;
+  // tile, twiddles, window and isqrt-start tables, wave sums
+  static constexpr size_t FIXED = TILE + (size_t)(N / 2) * 8 + (size_t)(N / 2 + 1) * 4 + (size_t)JLEN * 2 +
+                                  (size_t)(NT / 64 + 1) * 8 + 32;
+  static constexpr size_t HIST = (size_t)(HB_LDS + 1) * 4 + 3 * HB_LDS * 8 + HB_LDS * 4;
+  // dynamic LDS: three 64-bit sums, a count and a threshold per bin
+  static constexpr size_t dyn_bytes(int nb) { return M >= XB_TALL ? (size_t)nb * 32 + 8 : 0; }
+  static constexpr int CAP = M == XB_TALL && !TALL_OK ? 0 : (int)((LDS_BYTES - 8 - FIXED) / 32);
+  static constexpr size_t lds(int nb) { return FIXED + (M == XB_LDS ? HIST : dyn_bytes(nb)); }
+  // blocks per CU that the LDS holds
+  static constexpr int blocks(int nb) { return cmax(1, (int)(LDS_BYTES / lds(nb))); }
+  static constexpr int wpe() {
+    return M == XB_HBM ? 1 : cmax(1, cmin(4, blocks(2 * HB_LDS) * (NT / 64) / 4));
   }
 };
 
-template <int N, bool LH>
+template <int N, int M>
 __device__ __forceinline__ void xpass_bin_body(const Job& j, const float2* __restrict__ twg, int bx, int nbx) {
   const float2* __restrict__ spec = j.spec;
   const float* __restrict__ wtab = j.wtab;
   const int* __restrict__ thr_g = j.thr;
   const int* __restrict__ jst_g = j.jst;
   const int nb = j.nb;
-  using Cf = FFTCfg<N>;
-  constexpr int C = Cf::CX, NT = Cf::NTX, PS = C + 1;
+  using Cf = XBin<N, M>;
+  constexpr int C = Cf::C, NT = Cf::NT, PS = C + 1;
   constexpr int YT = N / C;
   constexpr int H = N / 2;
   // LDS: the tile, the S_0,2,4 histogram, the thresholds, the window factors of |k| <= N/2,
-  // the isqrt-start table and the first half of the twiddles (<= 80 KB at N = 512 so two
-  // blocks share a CU)
-  constexpr int JLEN = XBinLds<N>::JLEN;
+  // the isqrt-start table and the first half of the twiddles (<= 80 KB at N = 512 in XB_LDS
+  // so two blocks share a CU)
+  constexpr bool LH = M != XB_HBM;
+  constexpr bool LDYN = M >= XB_TALL;
+  constexpr int JLEN = Cf::JLEN;
   __shared__ float2 buf[N * PS];
-  __shared__ int thr_s[LH ? HB_LDS + 1 : 1];
-  __shared__ unsigned long long hs[LH ? 3 * HB_LDS : 1];   // fixed-point S_0, S_2, S_4
+  __shared__ int thr_st[M == XB_LDS ? HB_LDS + 1 : 1];
+  __shared__ unsigned long long hs_st[M == XB_LDS ? 3 * HB_LDS : 1];
   __shared__ double red_e[NT / 64 + 1];
-  __shared__ unsigned hc[LH ? HB_LDS : 1];   // stored modes binned per bin
+  __shared__ unsigned hc_st[M == XB_LDS ? HB_LDS : 1];
   __shared__ float wt_s[LH ? H + 1 : 1];
-  __shared__ short jst_s[LH ? JLEN : 1];   // bins < HB_LDS
+  __shared__ short jst_s[LH ? JLEN : 1];   // bins < CAP
   __shared__ float2 twh[N / 2];
+  extern __shared__ unsigned long long xbin_dyn[];
+  const int hstride = LDYN ? nb : HB_LDS;                           // bins per sum
+  unsigned long long* hs = LDYN ? xbin_dyn : hs_st;                 // fixed-point S_0, S_2, S_4
+  unsigned* hc = LDYN ? reinterpret_cast<unsigned*>(xbin_dyn + 3 * nb) : hc_st;   // stored modes binned per bin
+  int* thr_s = LDYN ? reinterpret_cast<int*>(hc + nb) : thr_st;
   const TwHalf<N> tw{twh};
   const int tid = threadIdx.x;
   for (int i = tid; i < N / 2; i += NT) twh[i] = twg[i];
   double* gpart = j.partials + (size_t)bx * nb * NACC;
   if constexpr (LH) {
     for (int i = tid; i <= nb; i += NT) thr_s[i] = thr_g[i];
-    for (int i = tid; i < 3 * HB_LDS; i += NT) hs[i] = 0ull;
-    for (int i = tid; i < HB_LDS; i += NT) hc[i] = 0u;
+    for (int i = tid; i < 3 * hstride; i += NT) hs[i] = 0ull;
+    for (int i = tid; i < hstride; i += NT) hc[i] = 0u;
     for (int i = tid; i <= H; i += NT) wt_s[i] = wtab[i];
     for (int i = tid; i < JLEN; i += NT) jst_s[i] = (short)jst_g[i];
   } else {
@@ -432,7 +462,7 @@ __device__ __forceinline__ void xpass_bin_body(const Job& j, const float2* __res
   // N = 128: the next tile's columns are loaded into registers while this one is transformed
   // and binned (for larger N the registers would spill or cost a block; at N = 64 a block
   // has a single tile)
-  constexpr bool XPF = LH && N == 128;
+  constexpr bool XPF = M == XB_LDS && N == 128;
   // tile loads: every lane keeps one column (NT is a multiple of C) and rows r0 + k RSTEP,
   // so its loads share one base address and all of them are in flight before any use
   static_assert(NT % C == 0, "tile lanes keep one column");
@@ -618,8 +648,8 @@ __device__ __forceinline__ void xpass_bin_body(const Job& j, const float2* __res
       const unsigned long long f4 = to_bin_fixed(a4, fscale);
       if constexpr (LH) {
         atomicAdd(&hs[cur], f0);
-        atomicAdd(&hs[HB_LDS + cur], f2);
-        atomicAdd(&hs[2 * HB_LDS + cur], f4);
+        atomicAdd(&hs[hstride + cur], f2);
+        atomicAdd(&hs[2 * hstride + cur], f4);
         atomicAdd(&hc[cur], (unsigned)cnt);
       } else {
         unsigned long long* g = reinterpret_cast<unsigned long long*>(gpart) + (size_t)cur * NACC;
@@ -688,25 +718,25 @@ __device__ __forceinline__ void xpass_bin_body(const Job& j, const float2* __res
     for (int i = tid; i < nb; i += NT) {
       unsigned long long* g = reinterpret_cast<unsigned long long*>(gpart) + (size_t)i * NACC;
       g[0] = hs[i];
-      g[1] = hs[HB_LDS + i];
-      g[2] = hs[2 * HB_LDS + i];
+      g[1] = hs[hstride + i];
+      g[2] = hs[2 * hstride + i];
       g[3] = (unsigned long long)hc[i];
     }
   }
 }
 
-template <int N, bool LH>
-__global__ void __launch_bounds__(FFTCfg<N>::NTX) __attribute__((amdgpu_waves_per_eu(XBinLds<N>::template wpe<LH>())))
+template <int N, int M>
+__global__ void __launch_bounds__((XBin<N, M>::NT)) __attribute__((amdgpu_waves_per_eu(XBin<N, M>::wpe())))
 k_xpass_bin(Job j, const float2* __restrict__ twg) {
-  xpass_bin_body<N, LH>(j, twg, blockIdx.x, gridDim.x);
+  xpass_bin_body<N, M>(j, twg, blockIdx.x, gridDim.x);
 }
 
-template <int N, bool LH>
-__global__ void __launch_bounds__(FFTCfg<N>::NTX) __attribute__((amdgpu_waves_per_eu(XBinLds<N>::template wpe<LH>())))
+template <int N, int M>
+__global__ void __launch_bounds__((XBin<N, M>::NT)) __attribute__((amdgpu_waves_per_eu(XBin<N, M>::wpe())))
 k_xpass_bin_jobs(const Job* __restrict__ jobs, const float2* __restrict__ twg) {
   const Job& j = jobs[blockIdx.y];
   if (!j.active) return;
-  xpass_bin_body<N, LH>(j, twg, blockIdx.x, gridDim.x);
+  xpass_bin_body<N, M>(j, twg, blockIdx.x, gridDim.x);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1456,35 +1486,109 @@ template <int N> struct FFTLaunch {
     if (!cap) cap = persistent_grid(k_ypass_jobs<N>, Cf::NTY, 1 << 30);
     return share(cap, njobs, YTILES);
   }
-  static int bin_jobs_grid(bool lh, int njobs) {
+  // histogram placement for nb bins (see XBin)
+  static int bin_mode(int nb) {
+    if (N != 1024 && nb <= HB_LDS) return XB_LDS;
+    if (nb <= XBin<N, XB_TALL>::CAP) return XB_TALL;
+    if (nb <= XBin<N, XB_WIDE>::CAP) return XB_WIDE;
+    return XB_HBM;
+  }
+  // resident blocks of the whole GPU for dynamic-LDS histograms of nb bins
+  template <int M> static int dyn_cap(int nb) {
+    int dev = 0;
+    (void)hipGetDevice(&dev);
+    return num_cus(dev) * XBin<N, M>::blocks(nb);
+  }
+  static int bin_jobs_grid(int nb, int njobs) {
     static int c_l = 0, c_g = 0;
-    int& cap = lh ? c_l : c_g;
-    if (!cap)
-      cap = lh ? persistent_grid(k_xpass_bin_jobs<N, true>, Cf::NTX, 1 << 30)
-               : persistent_grid(k_xpass_bin_jobs<N, false>, Cf::NTX, 1 << 30);
-    return share(cap, njobs, bin_grid(lh));
+    int cap = 0;
+    switch (bin_mode(nb)) {
+      case XB_LDS:
+        if constexpr (N != 1024) {
+          if (!c_l) c_l = persistent_grid(k_xpass_bin_jobs<N, XB_LDS>, Cf::NTX, 1 << 30);
+        }
+        cap = c_l;
+        break;
+      case XB_TALL: cap = dyn_cap<XB_TALL>(nb); break;
+      case XB_WIDE: cap = dyn_cap<XB_WIDE>(nb); break;
+      default:
+        if (!c_g) c_g = persistent_grid(k_xpass_bin_jobs<N, XB_HBM>, Cf::NTX, 1 << 30);
+        cap = c_g;
+    }
+    return share(cap, njobs, bin_grid(nb));
   }
   static int share(int cap, int njobs, int limit) {
     int g = (cap + njobs - 1) / (njobs < 1 ? 1 : njobs);
     if (g > limit) g = limit;
     return g < 1 ? 1 : g;
   }
-  static int bin_grid(bool lh) {
+  // blocks of one estimate that the partials hold rows for (the grid of the static and HBM
+  // histograms; the dynamic-LDS ones launch at most as many)
+  static int bin_grid(int nb) {
     static int g_l = 0, g_g = 0;
-    if (lh) {
-      if (!g_l) g_l = persistent_grid(k_xpass_bin<N, true>, Cf::NTX, XTILES);
+    if (nb <= HB_LDS) {
+      if constexpr (N != 1024) {
+        if (!g_l) g_l = persistent_grid(k_xpass_bin<N, XB_LDS>, Cf::NTX, XTILES);
+      } else {
+        g_l = dyn_cap<XB_LDS>(nb);
+      }
       return g_l;
     }
-    if (!g_g) g_g = persistent_grid(k_xpass_bin<N, false>, Cf::NTX, XTILES);
+    if (!g_g) g_g = persistent_grid(k_xpass_bin<N, XB_HBM>, Cf::NTX, XTILES);
     return g_g;
+  }
+  // blocks launched for one estimate
+  static int bin_blocks(int nb) {
+    const int m = bin_mode(nb), g = bin_grid(nb);
+    if (m == XB_TALL) return cmin(g, dyn_cap<XB_TALL>(nb));
+    if (m == XB_WIDE) return cmin(g, dyn_cap<XB_WIDE>(nb));
+    return g;
+  }
+  // raises a kernel's dynamic-LDS limit to its capacity, once (not again inside a capture)
+  template <int M, typename K> static int allow_bins(K kernel, bool& done) {
+    if (done) return PK_OK;
+    const int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                (int)XBin<N, M>::dyn_bytes(XBin<N, M>::CAP)),
+                            "LDS attribute");
+    done = e == PK_OK;
+    return e;
+  }
+  template <int M> static int launch_bin(const Job& j, const float2* tw, int grid, hipStream_t s) {
+    if constexpr (M >= XB_TALL) {
+      static bool done = false;
+      const int e = allow_bins<M>(k_xpass_bin<N, M>, done);
+      if (e) return e;
+    }
+    hipLaunchKernelGGL((k_xpass_bin<N, M>), dim3(grid), dim3(XBin<N, M>::NT), (XBin<N, M>::dyn_bytes(j.nb)), s, j,
+                       tw);
+    return PK_OK;
+  }
+  template <int M>
+  static int launch_bin_jobs(const Job* jobs, int njobs, int max_nb, int gx, const float2* tw, hipStream_t s) {
+    if constexpr (M >= XB_TALL) {
+      static bool done = false;
+      const int e = allow_bins<M>(k_xpass_bin_jobs<N, M>, done);
+      if (e) return e;
+    }
+    hipLaunchKernelGGL((k_xpass_bin_jobs<N, M>), dim3(gx, njobs), dim3(XBin<N, M>::NT),
+                       (XBin<N, M>::dyn_bytes(max_nb)), s, jobs, tw);
+    return PK_OK;
   }
   static int xpass_bin(const Job& j, const float2* tw, int grid, hipStream_t s) {
     StageTimer t(ST_XPASS_BIN, s);
-    if (j.nb <= HB_LDS)
-      hipLaunchKernelGGL((k_xpass_bin<N, true>), dim3(grid), dim3(Cf::NTX), 0, s, j, tw);
-    else
-      hipLaunchKernelGGL((k_xpass_bin<N, false>), dim3(grid), dim3(Cf::NTX), 0, s, j, tw);
-    return check_hip(hipGetLastError(), "x pass + bin launch");
+    int e = PK_OK;
+    switch (bin_mode(j.nb)) {
+      case XB_LDS:
+        if constexpr (N != 1024) e = launch_bin<XB_LDS>(j, tw, grid, s);
+        break;
+      case XB_TALL:
+        if constexpr (XBin<N, XB_TALL>::TALL_OK) e = launch_bin<XB_TALL>(j, tw, grid, s);
+        break;
+      case XB_WIDE: e = launch_bin<XB_WIDE>(j, tw, grid, s); break;
+      default: e = launch_bin<XB_HBM>(j, tw, grid, s);
+    }
+    return e ? e : check_hip(hipGetLastError(), "x pass + bin launch");
   }
   static int adjoint(const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh, hipStream_t s) {
     static int gx = 0, gy = 0, gz = 0;
@@ -1638,11 +1742,18 @@ template <int N> struct FFTLaunch {
   }
   static int xpass_bin_jobs(const Job* jobs, int njobs, int max_nb, int gx, const float2* tw, hipStream_t s) {
     StageTimer t(ST_XPASS_BIN, s);
-    if (max_nb <= HB_LDS)
-      hipLaunchKernelGGL((k_xpass_bin_jobs<N, true>), dim3(gx, njobs), dim3(Cf::NTX), 0, s, jobs, tw);
-    else
-      hipLaunchKernelGGL((k_xpass_bin_jobs<N, false>), dim3(gx, njobs), dim3(Cf::NTX), 0, s, jobs, tw);
-    return check_hip(hipGetLastError(), "batched x pass + bin launch");
+    int e = PK_OK;
+    switch (bin_mode(max_nb)) {
+      case XB_LDS:
+        if constexpr (N != 1024) e = launch_bin_jobs<XB_LDS>(jobs, njobs, max_nb, gx, tw, s);
+        break;
+      case XB_TALL:
+        if constexpr (XBin<N, XB_TALL>::TALL_OK) e = launch_bin_jobs<XB_TALL>(jobs, njobs, max_nb, gx, tw, s);
+        break;
+      case XB_WIDE: e = launch_bin_jobs<XB_WIDE>(jobs, njobs, max_nb, gx, tw, s); break;
+      default: e = launch_bin_jobs<XB_HBM>(jobs, njobs, max_nb, gx, tw, s);
+    }
+    return e ? e : check_hip(hipGetLastError(), "batched x pass + bin launch");
   }
 };
 
@@ -1733,7 +1844,7 @@ int ypass_jobs_grid(int n, int njobs) {
 
 int bin_jobs_grid(int n, int nb, int njobs) {
   switch (n) {
-#define PK_CASE(V) case V: return FFTLaunch<V>::bin_jobs_grid(nb <= HB_LDS, njobs);
+#define PK_CASE(V) case V: return FFTLaunch<V>::bin_jobs_grid(nb, njobs);
     PK_FOR_EACH_N(PK_CASE)
 #undef PK_CASE
   }
@@ -1742,7 +1853,16 @@ int bin_jobs_grid(int n, int nb, int njobs) {
 
 int bin_grid(int n, int nb) {
   switch (n) {
-#define PK_CASE(V) case V: return FFTLaunch<V>::bin_grid(nb <= HB_LDS);
+#define PK_CASE(V) case V: return FFTLaunch<V>::bin_grid(nb);
+    PK_FOR_EACH_N(PK_CASE)
+#undef PK_CASE
+  }
+  return 0;
+}
+
+int bin_blocks(int n, int nb) {
+  switch (n) {
+#define PK_CASE(V) case V: return FFTLaunch<V>::bin_blocks(nb);
     PK_FOR_EACH_N(PK_CASE)
 #undef PK_CASE
   }

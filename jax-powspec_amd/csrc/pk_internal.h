@@ -105,7 +105,8 @@ int fft_zpass(int n, const float* mesh, float2* spec, const float2* tw, const do
               double* sq_part,
               hipStream_t s);
 int fft_xpass(int n, float2* spec, const float2* tw, hipStream_t s);
-int bin_grid(int n, int nb);   // x-pass blocks of one estimate
+int bin_grid(int n, int nb);     // most x-pass blocks of one estimate (rows of the partials)
+int bin_blocks(int n, int nb);   // x-pass blocks launched for one estimate
 // blocks per job of a batch (y pass; x pass + binning, at most bin_grid(n, nb))
 int ypass_jobs_grid(int n, int njobs);
 int bin_jobs_grid(int n, int nb, int njobs);
