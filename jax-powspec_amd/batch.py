@@ -315,7 +315,7 @@ def powspec_batched(catalogues, *, tile="auto", graph: bool = True, device=None,
     fundamental bins), shot_noise, window, wrap, xmin/ymin/zmin.  tile: 'auto' (autotuned
     per mesh side on its own catalogues, cached), None (default rows per tile) or
     (1, ty, 0).  Every supported mesh side has a batched path (at 768 and 1024 with 16-row
-    tiles and the sort's per-key tables in HBM).
+    tiles).
     """
     device = _device.require_gpu(device)
     cats = list(catalogues)

@@ -331,7 +331,7 @@ int pk_scatter_workspace_size(int n, int64_t np, int stencil, const int* tile, s
   bool direct = false;
   int e = make_tile_geom(n, np, stencil, tile, &g, &direct);
   if (e) return e;
-  *bytes = scatter_workspace_bytes(g, direct, np);
+  *bytes = scatter_workspace_bytes(g, direct, n, np);
   return PK_OK;
 }
 
@@ -441,7 +441,7 @@ int carve_estimate(pk_plan* p, int64_t np, int stencil, const int* tile, int nb,
   w->mesh = w->fused ? nullptr : static_cast<float*>(take(n3 * sizeof(float)));
   w->spec = static_cast<float2*>(take((size_t)(n / 2 + 1) * n * n * sizeof(float2)));
   w->stats = static_cast<double*>(take(PK_STATS_LEN * sizeof(double)));
-  w->scatter_bytes = scatter_workspace_bytes(*g, *direct, np);
+  w->scatter_bytes = scatter_workspace_bytes(*g, *direct, n, np);
   w->scatter_ws = take(w->scatter_bytes);
   w->powspec_bytes = powspec_ws_bytes(n, nb);
   w->powspec_ws = take(w->powspec_bytes);
@@ -639,8 +639,8 @@ bool timing_suspended() { return t_capturing; }
 
 namespace {
 bool same_dims(const BatchDims& a, const BatchDims& b) {
-  return a.njobs == b.njobs && a.max_nblk == b.max_nblk && a.max_nkeys == b.max_nkeys && a.max_nb == b.max_nb &&
-         a.lds_keys == b.lds_keys && a.n == b.n && a.max_fblk == b.max_fblk;
+  return a.njobs == b.njobs && a.max_nblk == b.max_nblk && a.max_col == b.max_col && a.max_nb == b.max_nb &&
+         a.lds_keys == b.lds_keys && a.n == b.n && a.max_fblk == b.max_fblk && a.planes == b.planes && a.fine == b.fine;
 }
 
 int batch_geometry(int n, int64_t max_np, const int* tile, TileGeom* cap) {
@@ -666,6 +666,7 @@ SlotLayout slot_layout(int n, int64_t max_np, int max_nb, const TileGeom& cap, i
   L.scatter = off;
   Job cj{};
   cj.g = cap;
+  cj.a.n = n;
   cj.a.np = max_np;
   off += carve_scatter(cj, false, nullptr);
   L.bytes = align_up(off);
@@ -739,6 +740,7 @@ int pk_batch_create(pk_plan* p, int max_jobs, int64_t max_np, int max_nb, const 
     Job& j = b->slot[i];
     j = Job{};
     j.g = b->cap;
+    j.a.n = p->n;
     j.a.np = max_np;
     j.spec = reinterpret_cast<float2*>(base + L.spec);
     j.partials = reinterpret_cast<double*>(base + L.partials);
@@ -760,7 +762,7 @@ int pk_batch_create(pk_plan* p, int max_jobs, int64_t max_np, int max_nb, const 
   }
   b->cur = 0;
   b->njobs = 0;
-  b->dims = BatchDims{0, 0, 0, 0, 0, p->n, 1};
+  b->dims = BatchDims{0, 0, 0, 0, 0, p->n, 1, 0, 0};
   *out = b;
   return PK_OK;
 }
@@ -778,10 +780,7 @@ int pk_batch_set_jobs(pk_batch* b, int njobs, const pk_job* jobs, void* stream) 
     b->pending[k] = false;
   }
   Job* h = b->h_jobs[k];
-  BatchDims d{njobs, 1, 1, 1, 0, b->n, 1};
-  // capacity grids: one LDS table size for every refill (the capacity geometry's keys if
-  // they fit, else none), so captured launches repeat; jobs with more keys use HBM tables
-  const int cap_lds_keys = (size_t)b->cap.nkeys <= lds_table_keys() ? b->cap.nkeys : 0;
+  BatchDims d{njobs, 1, 1, 1, 0, b->n, 1, 0, 0};
   const int tile[3] = {1, b->cap.ty, 0};
   // counting chunk of a batch: about four rounds of blocks over the whole GPU for all its
   // particles (jobs of very different sizes balance), never more blocks per job than its slot holds
@@ -821,22 +820,25 @@ int pk_batch_set_jobs(pk_batch* b, int njobs, const pk_job* jobs, void* stream) 
     j.scale_stats = j.stats;
     j.sq_part = j.aux + 2;
     j.sq_n = 1;
-    h[i] = j;
     if (j.g.nblk > d.max_nblk) d.max_nblk = j.g.nblk;
-    if (j.g.nkeys > d.max_nkeys) d.max_nkeys = j.g.nkeys;
     if (fine_place_blocks(q.np) > d.max_fblk) d.max_fblk = fine_place_blocks(q.np);
     if (q.nb > d.max_nb) d.max_nb = q.nb;
-    if (b->flags & PK_BATCH_CAPACITY_GRIDS) {
-      if (j.g.nkeys > cap_lds_keys) h[i].g.gtab = 1;
-    } else if (!j.g.gtab && j.g.nkeys > d.lds_keys) {
-      d.lds_keys = j.g.nkeys;
-    }
+    // capacity grids: one set of launches for every refill, so captured ones repeat.  A job of
+    // fewer keys than the capacity geometry can take its way too.
+    if (b->flags & PK_BATCH_CAPACITY_GRIDS) j.g.sort = b->cap.sort;
+    h[i] = j;
+    if (sort_column_blocks(j.g, b->n) > d.max_col) d.max_col = sort_column_blocks(j.g, b->n);
+    if (count_columns(j.g, b->n) > d.lds_keys) d.lds_keys = count_columns(j.g, b->n);
+    d.planes |= j.g.sort == SORT_PLANES;
+    d.fine |= j.g.sort != SORT_KEYS;
   }
   if (b->flags & PK_BATCH_CAPACITY_GRIDS) {
     d.max_nblk = b->cap.nblk;
-    d.max_nkeys = b->cap.nkeys;
-    d.lds_keys = cap_lds_keys;
+    d.max_col = sort_column_blocks(b->cap, b->n);
+    d.lds_keys = count_columns(b->cap, b->n);
     d.max_fblk = fine_place_blocks(b->max_np);
+    d.planes = b->cap.sort == SORT_PLANES;
+    d.fine = b->cap.sort != SORT_KEYS;
   }
   hipStream_t s = as_stream(stream);
   if (njobs > 0) {

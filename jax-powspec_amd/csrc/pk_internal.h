@@ -35,9 +35,16 @@ struct TileGeom {
   int nblk;     // counting blocks
   int fixed;    // 1: deposit into 64-bit fixed-point LDS cells (ty * n * 8 bytes fit), 0: float
   unsigned ty_mul;   // ceil(2^32 / ty): y / ty = umulhi(y, ty_mul) for 0 <= y < n
-  int gtab;     // 1: the count and place kernels keep their per-key tables in HBM (the
-                // block's row of the count matrix, global atomics): nkeys too large for LDS
+  int sort;     // how the sort reaches the keys (see pk_scatter.hip):
 };
+// the count takes keys and the place sorts by them; the count takes keys and the place sorts by
+// x plane, then the fine pass by key; the count takes x planes, a pass per plane the keys
+enum { SORT_KEYS = 0, SORT_MIXED = 1, SORT_PLANES = 2 };
+// columns of the count matrix, and what the place sorts by: keys, or x planes and the irregular key
+__host__ __device__ inline int count_columns(const TileGeom& g, int n) {
+  return g.sort == SORT_PLANES ? n + 1 : g.nkeys;
+}
+__host__ __device__ inline int group_count(const TileGeom& g, int n) { return g.sort == SORT_KEYS ? g.nkeys : n + 1; }
 
 // LDS bytes up to which the deposit accumulates in 64-bit fixed point: gfx950 LDS
 // integer atomics run ~13x faster than float ones, and integer sums are order-independent
@@ -54,15 +61,17 @@ struct Job {
   TileGeom g;
   int active;            // 0: every kernel skips this job (unused batch slot)
   // sorted-deposit scratch
-  unsigned* mat;         // [nblk][nkeys] counts -> offsets inside each key
-  int* totals;           // [nkeys]
+  unsigned* mat;         // [nblk][columns] counts -> offsets inside each group
+  unsigned* pmat;        // [nblk][n + 1] the same of the x planes (SORT_MIXED; mat stays as counted)
+  int* totals;           // [columns]
+  int* ptotals;          // [n + 1] (SORT_MIXED)
   int* key_start;        // [nkeys + 1]
-  int* bsum;             // scan block sums
+  int* plane_start;      // [n + 2] (SORT_PLANES)
   double* wsum;          // [nblk] weight sums
   double* wmax;          // [nblk] max |w|
   double* aux;           // [AUX_LEN] fixed-point scale
   void* sorted;          // records
-  void* staged;          // records grouped by x plane only (the first placing pass)
+  void* staged;          // records grouped by x plane only
   unsigned* koff;        // [nkeys] records placed so far in each key (second pass)
   double* tile_mass;     // [ntiles]
   double* tile_sq;       // [ntiles] fused tiles' sums of (rho - c)^2 (nullptr: not reduced)
@@ -131,13 +140,13 @@ int bin_finalize_jobs(const Job* jobs, int njobs, int max_nb, int G, hipStream_t
 // validates/derives the tile geometry; tile == nullptr -> default rows per tile;
 // tile[0] == 0 -> direct global atomics; otherwise tile[1] = rows per tile
 int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g, bool* direct);
-// most keys whose count tables fit LDS (more: HBM tables)
-size_t lds_table_keys();
 // blocks of the second placing pass for np particles
 int fine_place_blocks(int64_t np);
+// blocks of the column scans
+int sort_column_blocks(const TileGeom& g, int n);
 // particles per counting block (clamped to the supported range) and the block count
 void set_chunk(TileGeom* g, int64_t np, int64_t chunk);
-size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int64_t np);
+size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int n, int64_t np);
 // points the sorted-deposit scratch of j into base (nullptr: sizes only); returns bytes
 size_t carve_scatter(Job& j, bool direct, void* base);
 // mesh_out == nullptr (tiled mode only): stop after sorting; the caller runs the fused
@@ -150,12 +159,13 @@ int mass_finalize(const Job& j, hipStream_t s);
 struct BatchDims {
   int njobs;
   int max_nblk;
-  int max_nkeys;
+  int max_col;    // blocks of the column scans of the largest job
   int max_nb;
-  int lds_keys;   // per-key LDS tables of count sized for this many keys (jobs with more
-                  // keys use HBM tables, gtab)
+  int lds_keys;   // LDS tables of the count kernel sized for this many columns
   int n;          // mesh side of every job
   int max_fblk;   // blocks of the second placing pass of the largest job
+  int planes;     // some job counts x planes (SORT_PLANES)
+  int fine;       // some job needs the fine pass (not SORT_KEYS)
 };
 int scatter_sort_jobs(const Job* jobs, const BatchDims& d, hipStream_t s);
 

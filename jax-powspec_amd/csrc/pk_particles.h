@@ -330,6 +330,20 @@ __device__ __forceinline__ float4 load_record(const void* sorted, size_t i, bool
   return r;
 }
 
+// Key of a record inside its x plane's keys (row_tile_key less the plane's first key): it
+// depends on the y coordinate alone.  Records of regular keys only.
+template <int ST = -1>
+__device__ __forceinline__ int row_key_in_plane(const ScatterArgs& a, const TileGeom& g, float py) {
+  const int stencil = ST >= 0 ? ST : a.stencil;
+  const int hy = home_cell(py, a.n, stencil);
+  const int yt = (int)__umulhi((unsigned)hy, g.ty_mul);
+  const int ly = hy - yt * g.ty;
+  int cls;
+  if (stencil == PK_STENCIL_TSC) cls = (ly == 0) ? 1 : ((ly == g.ty - 1) ? 2 : 0);
+  else cls = (ly == g.ty - 1) ? 1 : 0;
+  return yt * g.ncls + cls;
+}
+
 // Row-bundle tiles: tile (xt, yt) owns cells x = xt, y in [yt*ty, yt*ty + ty), all z.
 // Key = tile * ncls + y-class, where the y-class marks the tile rows whose stencil spills
 // into the neighbouring tile (CIC variants: 1 = last row; TSC: 1 = first, 2 = last row).
@@ -353,14 +367,8 @@ __device__ __forceinline__ int row_tile_key(const ScatterArgs& a, const TileGeom
     }
   }
   const int hx = home_cell(px, n, stencil);
-  const int hy = home_cell(py, n, stencil);
-  const int yt = (int)__umulhi((unsigned)hy, g.ty_mul);   // hy / ty
-  const int ly = hy - yt * g.ty;
-  int cls;
-  if (stencil == PK_STENCIL_TSC) cls = (ly == 0) ? 1 : ((ly == g.ty - 1) ? 2 : 0);
-  else cls = (ly == g.ty - 1) ? 1 : 0;
   if (plane) *plane = hx;
-  return (hx * g.nyt + yt) * g.ncls + cls;
+  return hx * g.nyt * g.ncls + row_key_in_plane<ST>(a, g, py);
 }
 
 // The x plane of row_tile_key's key (n for the irregular key), or -1 where it returns -1:

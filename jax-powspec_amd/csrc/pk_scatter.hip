@@ -3,22 +3,20 @@
 //
 // Sorted owner-computes deposit on row-bundle tiles (1 x ty x n cells, full z rows):
 //   1. count:  each block takes a chunk of particles (one block per CU) and histograms their
-//              keys (tile, y-class) in LDS, or in its row of the count matrix in HBM when
-//              the keys do not fit; the block's row of counts goes to a [blocks][keys]
-//              matrix.
-//   2. scan:   a column scan of the matrix gives every (block, key) its offset inside the
-//              key; an exclusive scan of the key totals gives the key starts.
-//   3. place, in two passes.  Keys are x-plane major, so the records of one x plane fill
-//              one contiguous range of the sorted order.
-//      a. coarse: the blocks re-read their chunk and write each record into its x plane's
-//              range (block offset = sum of the block's key offsets over the plane, plus an
-//              LDS rank).  A block appends to at most n + 1 runs, so the partly written
-//              128-byte lines of all blocks fit the L2 and leave it whole.
+//              keys (tile, y-class) in LDS, or their x planes when the keys do not fit.
+//   2. column: scans of the [blocks][groups] count matrix give every (block, group) its
+//              offset inside the group, and the totals.  Groups are what the place sorts by:
+//              keys on a small mesh, else x planes (keys are x-plane major).
+//   3. place:  the blocks scan the group totals into starts (each its own copy), re-read their
+//              chunk and write each record into its group's range (start + block offset + an
+//              LDS rank).  Groups = keys: the sort is done.  Groups = x planes:
+//      a. plane keys (only where the count could not take keys): one block per plane counts
+//                the plane's keys and scans them into key starts;
 //      b. fine:  blocks take consecutive segments of the plane-grouped records, histogram
-//              their keys over the segment's window of planes in LDS, reserve one run per
-//              key with a global atomic and write each key's records as one run.
-//              Owner-computes deposits sum in fixed point, so the order inside a key
-//              (atomic order) does not change any result.
+//                their keys over the segment's window of planes in LDS, reserve one run per
+//                key with a global atomic and write each key's records as one run.
+//      Owner-computes deposits sum in fixed point, so the order inside a key (atomic order)
+//      does not change any result.
 //   4. deposit: one block per tile stages its ty full rows in LDS (zeros or mesh_in), walks
 //              its own buckets plus the neighbour buckets that spill into it (the whole
 //              x - 1 / x + 1 tiles, the boundary-row classes of the y neighbours), adds every
@@ -76,12 +74,11 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
   const TileGeom g = j.g;
   const int tid = threadIdx.x;
   const bool packed = g.chunk <= 65535;
-  unsigned* row = j.mat + (size_t)bx * g.nkeys;
-  if (g.gtab) {   // per-key counters in the block's own row of the count matrix (HBM)
-    for (int k = tid; k < g.nkeys; k += CNT_NT) row[k] = 0u;
-    __threadfence();   // the zeros reach L2, where the atomics below add, before any adds
-  } else {
-    const int words = packed ? (g.nkeys + 1) >> 1 : g.nkeys;
+  const int ncol = count_columns(g, a.n);
+  unsigned* row = j.mat + (size_t)bx * ncol;
+  const bool planes = g.sort == SORT_PLANES;
+  {
+    const int words = packed ? (ncol + 1) >> 1 : ncol;
     for (int i = tid; i < words; i += CNT_NT) hist[i] = 0u;
   }
   if (tid == 0) wmax_bits = 0u;
@@ -105,10 +102,9 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
 #pragma unroll
     for (int u = 0; u < CNT_UNROLL; ++u) {
       if (i0 + (int64_t)u * CNT_NT >= hi) continue;
-      const int key = row_tile_key<ST>(a, g, px[u], py[u], pz[u]);
+      const int key = planes ? row_plane<ST>(a, px[u], py[u], pz[u]) : row_tile_key<ST>(a, g, px[u], py[u], pz[u]);
       if (key >= 0) {
-        if (g.gtab) atomicAdd(&row[key], 1u);
-        else if (packed) atomicAdd(&hist[key >> 1], 1u << (16 * (key & 1)));
+        if (packed) atomicAdd(&hist[key >> 1], 1u << (16 * (key & 1)));
         else atomicAdd(&hist[key], 1u);
         ws += (double)w[u];
         wm = fmaxf(wm, fabsf(w[u]));
@@ -118,8 +114,20 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
   atomicMax(&wmax_bits, __float_as_uint(wm));   // non-negative floats order like their bits
   __syncthreads();
   if (tid == 0) j.wmax[bx] = (double)__uint_as_float(wmax_bits);
-  if (!g.gtab)
-    for (int k = tid; k < g.nkeys; k += CNT_NT) row[k] = packed ? (hist[k >> 1] >> (16 * (k & 1))) & 0xffffu : hist[k];
+  auto count_of = [&](int k) { return packed ? (hist[k >> 1] >> (16 * (k & 1))) & 0xffffu : hist[k]; };
+  for (int k = tid; k < ncol; k += CNT_NT) row[k] = count_of(k);
+  if (g.sort == SORT_MIXED) {   // the block's x planes: sums over their keys
+    const int kpp = g.nyt * g.ncls;
+    for (int p = tid; p <= a.n; p += CNT_NT) {
+      unsigned sum = 0;
+      int q = p % kpp;   // rotated: the lanes' keys fall into different banks
+      for (int i = 0; p < a.n && i < kpp; ++i) {
+        sum += count_of(p * kpp + q);
+        q = q + 1 == kpp ? 0 : q + 1;
+      }
+      j.pmat[(size_t)bx * (a.n + 1) + p] = p < a.n ? sum : count_of(g.nkeys - 1);
+    }
+  }
   const double t = block_sum_f64(ws, red, CNT_NT);
   if (tid == 0) j.wsum[bx] = t;
 }
@@ -143,23 +151,23 @@ __global__ void __launch_bounds__(CNT_NT) k_bucket_count_jobs(const Job* __restr
 }
 
 // ------------------------------------------------------------------------------------
-// 2. column scan (offset of each block inside each key) + exclusive scan of key totals
+// 2. columns of the count matrix: offsets of the blocks inside each group, totals
 // ------------------------------------------------------------------------------------
 constexpr int COL_NT = 256;
-constexpr int COL_KEYS = 32;                  // keys per block: one 128-byte segment per row
-constexpr int COL_SUBS = COL_NT / COL_KEYS;   // threads per key, each over a run of rows
+constexpr int COL_KEYS = 32;                  // columns per block: one 128-byte segment per row
+constexpr int COL_SUBS = COL_NT / COL_KEYS;   // threads per column, each over a run of rows
 constexpr int COL_ROWS = 32;                  // rows per thread and pass (loads in flight)
 
-// Thread (sub, key) walks rows [sub * COL_ROWS, +COL_ROWS) of each pass of COL_SUBS *
-// COL_ROWS rows: the run sums of a key's threads meet in LDS, so one pass costs one round
-// trip to memory instead of a walk down the whole column.
-__device__ __forceinline__ void col_scan_body(const Job& j, int bx) {
+// Thread (sub, column) walks rows [sub * COL_ROWS, +COL_ROWS) of each pass of COL_SUBS *
+// COL_ROWS rows: the run sums of a column's threads meet in LDS, so one pass costs one round
+// trip to memory instead of a walk down the whole column.  SCAN: the counts become the
+// exclusive sums of the rows above; otherwise the matrix is only summed.
+template <bool SCAN>
+__device__ __forceinline__ void column_body(unsigned* mat, int ncol, int nblk, int* totals, int bx) {
   __shared__ unsigned part[COL_SUBS][COL_KEYS];
-  const int nkeys = j.g.nkeys, nblk = j.g.nblk;
-  unsigned* mat = j.mat;
   const int kk = threadIdx.x % COL_KEYS, sub = threadIdx.x / COL_KEYS;
   const int k = bx * COL_KEYS + kk;
-  const bool on = k < nkeys;
+  const bool on = k < ncol;
   unsigned carry = 0;
   for (int r0 = 0; r0 < nblk; r0 += COL_SUBS * COL_ROWS) {   // block-uniform
     const int rb = r0 + sub * COL_ROWS;
@@ -167,7 +175,7 @@ __device__ __forceinline__ void col_scan_body(const Job& j, int bx) {
     unsigned sum = 0;
 #pragma unroll
     for (int u = 0; u < COL_ROWS; ++u) {
-      c[u] = (on && rb + u < nblk) ? mat[(size_t)(rb + u) * nkeys + k] : 0u;
+      c[u] = (on && rb + u < nblk) ? mat[(size_t)(rb + u) * ncol + k] : 0u;
       sum += c[u];
     }
     part[sub][kk] = sum;
@@ -180,96 +188,32 @@ __device__ __forceinline__ void col_scan_body(const Job& j, int bx) {
       total += v;
     }
     __syncthreads();   // part is reused by the next pass
+    if constexpr (SCAN) {
 #pragma unroll
-    for (int u = 0; u < COL_ROWS; ++u) {
-      if (on && rb + u < nblk) {
-        mat[(size_t)(rb + u) * nkeys + k] = run;
-        run += c[u];
+      for (int u = 0; u < COL_ROWS; ++u) {
+        if (on && rb + u < nblk) {
+          mat[(size_t)(rb + u) * ncol + k] = run;
+          run += c[u];
+        }
       }
     }
     carry += total;
   }
-  if (on && sub == 0) {
-    j.totals[k] = (int)carry;
-    j.koff[k] = 0u;   // the fine placing pass counts each key's records from zero
-  }
-}
-__global__ void __launch_bounds__(COL_NT) k_col_scan(Job j) { col_scan_body(j, blockIdx.x); }
-__global__ void __launch_bounds__(COL_NT) k_col_scan_jobs(const Job* __restrict__ jobs) {
-  PK_JOB_OR_RETURN(jobs, (j.g.nkeys + COL_KEYS - 1) / COL_KEYS);
-  col_scan_body(j, blockIdx.x);
+  if (on && sub == 0) totals[k] = (int)carry;
 }
 
-constexpr int SCAN_NT = 1024;
-constexpr int SCAN_PER = 4;
-constexpr int SCAN_BLOCK = SCAN_NT * SCAN_PER;
-
-// wave scans with shuffles, then the wave totals (two barriers)
-__device__ int block_exclusive_scan(int v, int* sh, int& total) {
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  int incl = v;
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int t = __shfl_up(incl, off, 64);
-    if (lane >= off) incl += t;
-  }
-  if (lane == 63) sh[w] = incl;
-  __syncthreads();
-  int before = 0, tot = 0;
-#pragma unroll
-  for (int i = 0; i < SCAN_NT / 64; ++i) {
-    const int x = sh[i];
-    if (i < w) before += x;
-    tot += x;
-  }
-  total = tot;
-  __syncthreads();
-  return before + incl - v;
-}
-
-// key totals -> key starts: local scans of SCAN_BLOCK keys, a scan of the block sums, add
-__device__ __forceinline__ void scan_local_body(const Job& j, int bx) {
-  __shared__ int sh[SCAN_NT];
-  const int n = j.g.nkeys;
-  const int* in = j.totals;
-  int* out = j.key_start;
-  const int base = bx * SCAN_BLOCK + threadIdx.x * SCAN_PER;
-  int v[SCAN_PER];
-  int s = 0;
-#pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k) {
-    v[k] = (base + k < n) ? in[base + k] : 0;
-    s += v[k];
-  }
-  int total;
-  int run = block_exclusive_scan(s, sh, total);
-#pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k) {
-    if (base + k < n) out[base + k] = run;
-    run += v[k];
-  }
-  if (threadIdx.x == 0) j.bsum[bx] = total;
-}
-__global__ void __launch_bounds__(SCAN_NT) k_scan_local(Job j) { scan_local_body(j, blockIdx.x); }
-__global__ void __launch_bounds__(SCAN_NT) k_scan_local_jobs(const Job* __restrict__ jobs) {
-  PK_JOB_OR_RETURN(jobs, (j.g.nkeys + SCAN_BLOCK - 1) / SCAN_BLOCK);
-  scan_local_body(j, blockIdx.x);
-}
-
-// key_start[nkeys] = the records' total; sums the weight partials into stats[3] =
-// sum(w) / n^3 and sets the fixed-point scale aux[0] = S, aux[1] = 1 / S from max |w|.
-// Every thread of the block must call it.
-__device__ __forceinline__ void scan_finish_body(const Job& j, int total) {
-  __shared__ double shd[SCAN_NT];
+// sums the weight partials into stats[3] = sum(w) / n^3 and sets the fixed-point scale
+// aux[0] = S, aux[1] = 1 / S from max |w|
+__device__ __forceinline__ void weight_stats_body(const Job& j) {
+  __shared__ double shd[COL_NT / 64 + 1];
   __shared__ unsigned long long wmax_bits;
-  if (threadIdx.x == 0) j.key_start[j.g.nkeys] = total;
   double ws = 0.0, wm = 0.0;
   if (threadIdx.x == 0) wmax_bits = 0ull;
-  for (int i = threadIdx.x; i < j.g.nblk; i += SCAN_NT) {
+  for (int i = threadIdx.x; i < j.g.nblk; i += COL_NT) {
     ws += j.wsum[i];
     wm = fmax(wm, j.wmax[i]);
   }
-  const double t = block_sum_f64_waves<SCAN_NT>(ws, shd);   // ends with a barrier
+  const double t = block_sum_f64_waves<COL_NT>(ws, shd);   // ends with a barrier
   atomicMax(&wmax_bits, (unsigned long long)__double_as_longlong(wm));
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -284,38 +228,26 @@ __device__ __forceinline__ void scan_finish_body(const Job& j, int total) {
     j.aux[1] = ldexp(1.0, e - 30);
   }
 }
-// all keys in one local block: the local scan, then the finish (no add pass follows)
-__global__ void __launch_bounds__(SCAN_NT) k_scan_single(Job j) {
-  scan_local_body(j, 0);
-  __syncthreads();
-  scan_finish_body(j, j.bsum[0]);
-}
 
-// Block bx adds the sum of the block sums before it to its keys' local starts (each block
-// sums that short prefix itself, so no separate scan of the block sums runs); block 0 also
-// finishes (the records' total and the weight statistics).
-__device__ __forceinline__ void scan_add_body(const Job& j, int bx) {
-  __shared__ int sh[SCAN_NT / 64];
-  const int n = j.g.nkeys;
-  const int nb2 = (n + SCAN_BLOCK - 1) / SCAN_BLOCK;
-  const int* bsum = j.bsum;
-  const int upto = bx == 0 ? nb2 : bx;   // block 0: every block sum (the total); else those before bx
-  int s = 0;
-  for (int i = threadIdx.x; i < upto; i += SCAN_NT) s += bsum[i];
-  int sum;
-  (void)block_exclusive_scan(s, sh, sum);
-  int* out = j.key_start;
-  const int base = bx * SCAN_BLOCK + threadIdx.x * SCAN_PER;
-  const int add = bx == 0 ? 0 : sum;
-#pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k)
-    if (base + k < n) out[base + k] += add;
-  if (bx == 0) scan_finish_body(j, sum);   // block-uniform
+// blocks: the groups' columns, the keys' columns (sums only) where the groups are the planes
+// of counted keys, and one for the weights
+__host__ __device__ inline int column_blocks(const TileGeom& g, int n) {
+  return (group_count(g, n) + COL_KEYS - 1) / COL_KEYS +
+         (g.sort == SORT_MIXED ? (g.nkeys + COL_KEYS - 1) / COL_KEYS : 0) + 1;
 }
-__global__ void __launch_bounds__(SCAN_NT) k_scan_add(Job j) { scan_add_body(j, blockIdx.x); }
-__global__ void __launch_bounds__(SCAN_NT) k_scan_add_jobs(const Job* __restrict__ jobs) {
-  PK_JOB_OR_RETURN(jobs, (j.g.nkeys + SCAN_BLOCK - 1) / SCAN_BLOCK);
-  scan_add_body(j, blockIdx.x);
+__device__ __forceinline__ void columns_body(const Job& j, int bx) {
+  const TileGeom& g = j.g;
+  const int G = group_count(g, j.a.n);
+  const int ng = (G + COL_KEYS - 1) / COL_KEYS;
+  if (bx == column_blocks(g, j.a.n) - 1) weight_stats_body(j);
+  else if (bx >= ng) column_body<false>(j.mat, g.nkeys, g.nblk, j.totals, bx - ng);
+  else if (g.sort == SORT_MIXED) column_body<true>(j.pmat, G, g.nblk, j.ptotals, bx);
+  else column_body<true>(j.mat, G, g.nblk, j.totals, bx);
+}
+__global__ void __launch_bounds__(COL_NT) k_columns(Job j) { columns_body(j, blockIdx.x); }
+__global__ void __launch_bounds__(COL_NT) k_columns_jobs(const Job* __restrict__ jobs) {
+  PK_JOB_OR_RETURN(jobs, column_blocks(j.g, j.a.n));
+  columns_body(j, blockIdx.x);
 }
 
 // ------------------------------------------------------------------------------------
@@ -359,18 +291,70 @@ __device__ __forceinline__ unsigned block_scan_apply(const unsigned* a, int len,
 }
 
 // ------------------------------------------------------------------------------------
-// 3a. coarse place: x-plane start + block offset inside the plane + LDS rank
+// 3. place by group: group start + block offset inside the group + LDS rank
 // ------------------------------------------------------------------------------------
 constexpr int PLACE_PER = 7;                     // most particles per thread and round
-constexpr size_t PLACE_LDS = 150 * 1024;         // tables + staging of the coarse pass
+constexpr size_t PLACE_LDS = 150 * 1024;         // tables + staging
 // particles per round: 20 staged bytes each (x, y, z, w, destination) next to three tables
-// of n + 1 words, a multiple of the block size
-__host__ __device__ constexpr int place_round(int n) {
-  return (int)((PLACE_LDS - 12 * (size_t)(n + 1)) / 20) / CNT_NT * CNT_NT > CNT_NT * PLACE_PER
+// of one word per group, a multiple of the block size
+__host__ __device__ constexpr int place_round(int groups) {
+  return (int)((PLACE_LDS - 12 * (size_t)groups) / 20) / CNT_NT * CNT_NT > CNT_NT * PLACE_PER
              ? CNT_NT * PLACE_PER
-             : (int)((PLACE_LDS - 12 * (size_t)(n + 1)) / 20) / CNT_NT * CNT_NT;
+             : (int)((PLACE_LDS - 12 * (size_t)groups) / 20) / CNT_NT * CNT_NT;
 }
-size_t place_lds(int n) { return 12 * ((size_t)n + 1) + 20 * (size_t)place_round(n); }
+size_t place_lds(int groups) { return 12 * (size_t)groups + 20 * (size_t)place_round(groups); }
+
+// Every block scans the group totals into its own group starts (no launch and no round trip
+// between the column scan and the place) and adds its offsets: dest[] (lcnt: scratch).  The
+// starts that later passes read go to memory too: key_start (groups = keys: by block 0;
+// planes of counted keys: each block the keys of some planes), or plane_start.
+template <int ST>
+__device__ __forceinline__ void place_starts(const Job& j, int bx, unsigned* dest, unsigned* lcnt, unsigned* wtot) {
+  const TileGeom& g = j.g;
+  const int n = j.a.n, G = group_count(g, n), tid = threadIdx.x;
+  const unsigned* row = (g.sort == SORT_MIXED ? j.pmat : j.mat) + (size_t)bx * G;
+  const int* tot = g.sort == SORT_MIXED ? j.ptotals : j.totals;
+  for (int i = tid; i < G; i += CNT_NT) {
+    lcnt[i] = (unsigned)tot[i];
+    dest[i] = row[i];
+  }
+  __syncthreads();
+  int* starts = g.sort == SORT_KEYS ? j.key_start : j.plane_start;
+  const bool write = bx == 0 && g.sort != SORT_MIXED;
+  const unsigned all = block_scan_apply<CNT_NT>(lcnt, G, wtot, [&](int i, unsigned, unsigned e) {
+    dest[i] += e;
+    lcnt[i] = e;
+    if (write) starts[i] = (int)e;
+  });
+  if (write && tid == 0) starts[G] = (int)all;
+  if (g.sort == SORT_MIXED) {
+    __syncthreads();   // lcnt: plane starts
+    const int kpp = g.nyt * g.ncls, lane = tid & 63;
+    constexpr int NW = CNT_NT / 64;
+    // one wave per plane; the planes are dealt over the blocks' waves
+    for (int p = bx * NW + (tid >> 6); p <= n; p += g.nblk * NW) {
+      const int k0 = p * kpp, kn = p < n ? kpp : 1;
+      int run = (int)lcnt[p];
+      for (int q0 = 0; q0 < kn; q0 += 64) {
+        const int q = q0 + lane;
+        const int c = q < kn ? j.totals[k0 + q] : 0;
+        int incl = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int v = __shfl_up(incl, off, 64);
+          if (lane >= off) incl += v;
+        }
+        if (q < kn) {
+          j.key_start[k0 + q] = run + incl - c;
+          j.koff[k0 + q] = 0u;   // the fine pass counts each key's records from zero
+        }
+        run += __shfl(incl, 63, 64);
+      }
+      if (p == n && lane == 0) j.key_start[g.nkeys] = run;
+    }
+  }
+  __syncthreads();   // dest complete, lcnt free
+}
 
 template <int AOS, int W, int ST = -1>
 __device__ __forceinline__ void bucket_place_body(const Job& j, int bx, unsigned* wtot) {
@@ -378,31 +362,18 @@ __device__ __forceinline__ void bucket_place_body(const Job& j, int bx, unsigned
   const ScatterArgs a = j.a;
   const TileGeom g = j.g;
   const int tid = threadIdx.x;
-  const int G = a.n + 1;            // x planes, then the irregular key
-  const int S = place_round(a.n);   // particles per round
-  unsigned* dest = lds;             // next write position of each plane for this block
-  unsigned* lcnt = lds + G;         // the round's count, then local start, of each plane
-  unsigned* delta = lds + 2 * G;    // global position - local slot, per plane
+  const int G = group_count(g, a.n);
+  const bool by_key = g.sort == SORT_KEYS;
+  const int S = place_round(G);     // particles per round
+  unsigned* dest = lds;             // next write position of each group for this block
+  unsigned* lcnt = lds + G;         // the round's count, then local start, of each group
+  unsigned* delta = lds + 2 * G;    // global position - local slot, per group
   float* sx = reinterpret_cast<float*>(lds + 3 * G);
   float* sy = sx + S;
   float* sz = sy + S;
   float* sw = sz + S;
   unsigned* sd = reinterpret_cast<unsigned*>(sw + S);   // global position of each slot
-  const unsigned kpp = (unsigned)(g.nyt * g.ncls);
-  {
-    // plane start + the records of this plane in earlier blocks (the sum of this block's
-    // offsets over the plane's keys): one wave per plane
-    const unsigned* row = j.mat + (size_t)bx * g.nkeys;
-    const int wv = tid >> 6, ln = tid & 63;
-    for (int i = wv; i < G; i += CNT_NT / 64) {
-      const int k0 = i * (int)kpp, k1 = i < a.n ? k0 + (int)kpp : g.nkeys;
-      unsigned sum = 0;
-      for (int k = k0 + ln; k < k1; k += 64) sum += row[k];
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-      if (ln == 0) dest[i] = (unsigned)j.key_start[k0] + sum;
-    }
-  }
+  void* out = by_key ? j.sorted : j.staged;
   const int64_t lo = (int64_t)bx * g.chunk;
   const int64_t hi = min(lo + (int64_t)g.chunk, a.np);
   const bool has_w = a.w != nullptr;
@@ -416,14 +387,17 @@ __device__ __forceinline__ void bucket_place_body(const Job& j, int bx, unsigned
     for (int u = 0; u < PLACE_PER; ++u)
       load_particle<AOS, W, true>(a, min(r0 + (int64_t)u * CNT_NT + tid, hi - 1), x[u], y[u], z[u], ww[u]);
   };
+  if (lo < hi) load_round(lo, px, py, pz, w);
+  place_starts<ST>(j, bx, dest, lcnt, wtot);
   if (lo >= hi) return;   // whole block: an empty chunk
-  load_round(lo, px, py, pz, w);
   for (int64_t r0 = lo; r0 < hi; r0 += S) {   // block-uniform
     int pl[PLACE_PER];
 #pragma unroll
     for (int u = 0; u < PLACE_PER; ++u) {
       const int64_t i = r0 + (int64_t)u * CNT_NT + tid;
-      pl[u] = (u * CNT_NT < S && i < hi) ? row_plane<ST>(a, px[u], py[u], pz[u]) : -1;
+      pl[u] = (u * CNT_NT >= S || i >= hi) ? -1
+              : by_key                   ? row_tile_key<ST>(a, g, px[u], py[u], pz[u])
+                                         : row_plane<ST>(a, px[u], py[u], pz[u]);
     }
     float nx[PLACE_PER], ny[PLACE_PER], nz[PLACE_PER], nw[PLACE_PER];
     load_round(r0 + S, nx, ny, nz, nw);
@@ -436,7 +410,7 @@ __device__ __forceinline__ void bucket_place_body(const Job& j, int bx, unsigned
     __syncthreads();
     const unsigned m = block_scan_apply<CNT_NT>(lcnt, G, wtot, [&](int p, unsigned c, unsigned e) {
       lcnt[p] = e;
-      if (c) {   // this thread alone owns plane p here
+      if (c) {   // this thread alone owns group p here
         const unsigned b = dest[p];
         dest[p] = b + c;
         delta[p] = b - e;
@@ -454,7 +428,7 @@ __device__ __forceinline__ void bucket_place_body(const Job& j, int bx, unsigned
         sd[slot] = delta[pl[u]] + slot;
       }
     __syncthreads();
-    for (int q = tid; q < (int)m; q += CNT_NT) store_record(j.staged, sd[q], has_w, sx[q], sy[q], sz[q], sw[q]);
+    for (int q = tid; q < (int)m; q += CNT_NT) store_record(out, sd[q], has_w, sx[q], sy[q], sz[q], sw[q]);
 #pragma unroll
     for (int u = 0; u < PLACE_PER; ++u) {
       px[u] = nx[u];
@@ -500,6 +474,54 @@ template <int AOS, int W, int ST> struct CountK { static constexpr void (*k)(Job
 template <int AOS, int W, int ST> struct PlaceK { static constexpr void (*k)(Job) = k_bucket_place<AOS, W, ST>; };
 
 // ------------------------------------------------------------------------------------
+// 3a. the keys of one x plane's records, counted in LDS and scanned into key starts (where the
+// count took planes; block n takes the irregular key)
+// ------------------------------------------------------------------------------------
+constexpr int PKEY_NT = 1024;
+constexpr int PKEY_UNROLL = 8;
+__device__ __forceinline__ void plane_keys_body(const Job& j, int p) {
+  extern __shared__ unsigned lds[];   // [keys per plane]
+  __shared__ unsigned wtot[PKEY_NT / 64];
+  const ScatterArgs a = j.a;
+  const TileGeom g = j.g;
+  const int tid = threadIdx.x;
+  const int lo = j.plane_start[p], hi = j.plane_start[p + 1];
+  if (p == a.n) {
+    if (tid == 0) {
+      j.key_start[g.nkeys - 1] = lo;
+      j.key_start[g.nkeys] = hi;
+      j.koff[g.nkeys - 1] = 0u;
+    }
+    return;
+  }
+  const int kpp = g.nyt * g.ncls;
+  for (int i = tid; i < kpp; i += PKEY_NT) lds[i] = 0u;
+  __syncthreads();
+  const int stride = a.w != nullptr ? 4 : 3;
+  const float* y = static_cast<const float*>(j.staged) + 1;   // y of record i at y[i stride]
+  for (int64_t i0 = lo + tid; i0 < hi; i0 += PKEY_NT * PKEY_UNROLL) {
+    float py[PKEY_UNROLL];
+#pragma unroll
+    for (int u = 0; u < PKEY_UNROLL; ++u) py[u] = y[min(i0 + u * PKEY_NT, (int64_t)hi - 1) * stride];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < PKEY_UNROLL; ++u)
+      if (i0 + u * PKEY_NT < hi) atomicAdd(&lds[row_key_in_plane(a, g, py[u])], 1u);
+  }
+  __syncthreads();
+  block_scan_apply<PKEY_NT>(lds, kpp, wtot, [&](int q, unsigned, unsigned e) {
+    j.key_start[p * kpp + q] = lo + (int)e;
+    j.koff[p * kpp + q] = 0u;
+  });
+}
+__global__ void __launch_bounds__(PKEY_NT) k_plane_keys(Job j) { plane_keys_body(j, blockIdx.x); }
+__global__ void __launch_bounds__(PKEY_NT) k_plane_keys_jobs(const Job* __restrict__ jobs) {
+  const Job& j = jobs[blockIdx.y];
+  if (!j.active || j.g.sort != SORT_PLANES) return;
+  plane_keys_body(j, blockIdx.x);
+}
+
+// ------------------------------------------------------------------------------------
 // 3b. fine place: a segment of the plane-grouped records -> one run per (segment, key)
 // ------------------------------------------------------------------------------------
 constexpr int FINE_NT = 256;                      // small blocks, several per CU: their
@@ -534,9 +556,7 @@ __device__ __forceinline__ void fine_place_body(const Job& j, int bx) {
   // the records are grouped by plane, so the first and last records bound the segment's planes
   if (tid < 2) {
     const float4 r = load_record(j.staged, (size_t)(tid == 0 ? s0 : s1 - 1), has_w);
-    int plane = 0;
-    (void)row_tile_key<ST>(a, g, r.x, r.y, r.z, &plane);
-    win[tid] = plane;
+    win[tid] = row_plane<ST>(a, r.x, r.y, r.z);
   }
   float4 r[FINE_PER];
   int key[FINE_PER];
@@ -548,7 +568,7 @@ __device__ __forceinline__ void fine_place_body(const Job& j, int bx) {
   for (int u = 0; u < FINE_PER; ++u) {
     const int64_t i = s0 + tid + (int64_t)u * FINE_NT;
     r[u].w = record_weight(r[u], has_w);
-    key[u] = i < s1 ? row_tile_key<ST>(a, g, r[u].x, r[u].y, r[u].z) : -1;   // the key the coarse pass saw
+    key[u] = i < s1 ? row_tile_key<ST>(a, g, r[u].x, r[u].y, r[u].z) : -1;   // of the plane the place saw
   }
   __syncthreads();
   const int kbase = win[0] * (int)kpp;
@@ -593,7 +613,7 @@ template <int ST>
 __global__ void __launch_bounds__(FINE_NT) k_fine_place(Job j) { fine_place_body<ST>(j, blockIdx.x); }
 __global__ void __launch_bounds__(FINE_NT) k_fine_place_jobs(const Job* __restrict__ jobs) {
   const Job& j = jobs[blockIdx.y];
-  if (!j.active) return;
+  if (!j.active || j.g.sort == SORT_KEYS) return;
   fine_place_body(j, blockIdx.x);
 }
 
@@ -716,7 +736,19 @@ __global__ void __launch_bounds__(MASS_NT) k_mass_finalize(Job j, int ntiles) { 
 // host side
 // ------------------------------------------------------------------------------------
 constexpr size_t LDS_MAX = 160 * 1024;
-constexpr size_t LDS_TABLE_MAX = LDS_MAX - 16384;   // per-key tables of count / place in LDS
+// Sort by the keys themselves up to this many (SORT_KEYS): the fine pass is saved, but a round's
+// records spread over more runs and more of the LDS goes to tables.  Whole estimates, us, by key
+// against by plane and then by key (SORT_MIXED): 1025 keys (128^3) 72 / 80 with 1e6 particles
+// and 585 / 668 with 3e7; 3457 keys (192^3 TSC) 235 / 242 with 5e6 and 996 / 1009 with 3e7;
+// 4097 keys (256^3) 136 / 138 with 1e6 but 526 / 516 with 2e7.
+constexpr long SORT_KEYS_MAX = 4000;
+// Count keys up to this many (SORT_MIXED: 32-bit counters in LDS), x planes beyond (n = 768 and
+// 1024, tiles of few rows).  Counting planes alone reads the staged records once more for their
+// keys: 384^3 with 3e7 particles took 1101 us that way against 1004.  Keys that do not fit LDS
+// went to per-block tables in HBM before (global atomics): 1314 us of counting and 77 us of
+// column scan at 1024^3 with 3e7 particles, against 70 + 6 us and 95 us for the plane keys.
+constexpr long COUNT_KEYS_MAX = (LDS_MAX - 16384) / 4;
+constexpr long KEYS_MAX = 1L << 24;
 constexpr int CHUNK_MIN = 4096;          // smallest counting chunk (small catalogues)
 constexpr int CHUNK_MAX = 1 << 22;       // largest (32-bit LDS counters above 65535)
 
@@ -733,8 +765,6 @@ void set_chunk(TileGeom* g, int64_t np, int64_t chunk) {
   g->nblk = (int)((np + chunk - 1) / chunk);
   if (g->nblk < 1) g->nblk = 1;
 }
-
-size_t lds_table_keys() { return LDS_TABLE_MAX / 4; }
 
 int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g, bool* direct) {
   *direct = false;
@@ -769,9 +799,7 @@ int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g,
   g->ntiles = (int)ntiles;
   g->nkeys = (int)nkeys;
   g->fixed = (size_t)ty * n * 8 <= FIXED_LDS_MAX ? 1 : 0;
-  // per-key tables of the count and place kernels: LDS when they fit, else the block's
-  // row of the count matrix in HBM
-  g->gtab = (size_t)nkeys * 4 > LDS_TABLE_MAX ? 1 : 0;
+  g->sort = nkeys <= SORT_KEYS_MAX ? SORT_KEYS : nkeys <= COUNT_KEYS_MAX ? SORT_MIXED : SORT_PLANES;
   // one counting / placing block per CU when the catalogue is large (a second, partial
   // round of blocks would cost a whole round), at least CHUNK_MIN particles per block
   int dev = 0;
@@ -779,8 +807,7 @@ int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g,
   const int64_t ncu = num_cus(dev);
   set_chunk(g, np, (np + ncu - 1) / ncu);
   if (g->nblk < 1) g->nblk = 1;
-  if ((long)g->nkeys > (long)SCAN_BLOCK * SCAN_BLOCK || g->nblk > SCAN_BLOCK * SCAN_BLOCK)
-    return set_error(PK_E_INVALID, "too many buckets");
+  if (nkeys > KEYS_MAX) return set_error(PK_E_INVALID, "too many buckets");
   return PK_OK;
 }
 
@@ -807,11 +834,15 @@ int allow_lds(K kernel, size_t bytes) {
   return e;
 }
 
-size_t hist_lds(const TileGeom& g) {
-  if (g.gtab) return 0;
-  return g.chunk <= 65535 ? (size_t)((g.nkeys + 1) / 2) * 4 : (size_t)g.nkeys * 4;
+size_t hist_lds(const TileGeom& g, int n) {
+  const size_t ncol = (size_t)count_columns(g, n);
+  return g.chunk <= 65535 ? (ncol + 1) / 2 * 4 : ncol * 4;
 }
+// keys of one plane: at most 3 n / 2 words (24 KB at n = 4096)
+size_t plane_keys_lds(const TileGeom& g) { return (size_t)g.nyt * g.ncls * sizeof(unsigned); }
 }  // namespace
+
+int sort_column_blocks(const TileGeom& g, int n) { return column_blocks(g, n); }
 
 size_t carve_scatter(Job& j, bool direct, void* base) {
   size_t off = 0;
@@ -826,9 +857,11 @@ size_t carve_scatter(Job& j, bool direct, void* base) {
   if (!j.stats) j.stats = st;
   if (!direct) {
     j.mat = static_cast<unsigned*>(take((size_t)g.nblk * g.nkeys * sizeof(unsigned)));
+    j.pmat = static_cast<unsigned*>(take((size_t)g.nblk * (j.a.n + 1) * sizeof(unsigned)));
     j.totals = static_cast<int*>(take((size_t)g.nkeys * sizeof(int)));
+    j.ptotals = static_cast<int*>(take(((size_t)j.a.n + 1) * sizeof(int)));
     j.key_start = static_cast<int*>(take(((size_t)g.nkeys + 1) * sizeof(int)));
-    j.bsum = static_cast<int*>(take((size_t)SCAN_BLOCK * sizeof(int)));
+    j.plane_start = static_cast<int*>(take(((size_t)j.a.n + 2) * sizeof(int)));
     j.wsum = static_cast<double*>(take((size_t)g.nblk * sizeof(double)));
     j.wmax = static_cast<double*>(take((size_t)g.nblk * sizeof(double)));
     j.aux = static_cast<double*>(take(AUX_LEN * sizeof(double)));
@@ -841,10 +874,11 @@ size_t carve_scatter(Job& j, bool direct, void* base) {
   return off;
 }
 
-size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int64_t np) {
+size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int n, int64_t np) {
   Job j{};
   j.g = g;
   j.a.np = np;
+  j.a.n = n;
   return carve_scatter(j, direct, nullptr);
 }
 
@@ -884,7 +918,7 @@ int scatter_run(Job& j, bool direct, const float* mesh_in, float* mesh_out, void
   }
   {
     StageTimer t(ST_SORT_COUNT, s);
-    const size_t lds = hist_lds(g);
+    const size_t lds = hist_lds(g, a.n);
     const auto kc = pick_aw<CountK>(a);
     int e = allow_lds(kc, lds);
     if (e) return e;
@@ -894,20 +928,13 @@ int scatter_run(Job& j, bool direct, const float* mesh_in, float* mesh_out, void
   }
   {
     StageTimer t(ST_SCAN, s);
-    hipLaunchKernelGGL(k_col_scan, dim3((g.nkeys + COL_KEYS - 1) / COL_KEYS), dim3(COL_NT), 0, s, j);
-    const int nb2 = (g.nkeys + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    if (nb2 == 1) {
-      hipLaunchKernelGGL(k_scan_single, dim3(1), dim3(SCAN_NT), 0, s, j);
-    } else {
-      hipLaunchKernelGGL(k_scan_local, dim3(nb2), dim3(SCAN_NT), 0, s, j);
-      hipLaunchKernelGGL(k_scan_add, dim3(nb2), dim3(SCAN_NT), 0, s, j);
-    }
+    hipLaunchKernelGGL(k_columns, dim3(column_blocks(g, a.n)), dim3(COL_NT), 0, s, j);
     int e = check_hip(hipGetLastError(), "scan launch");
     if (e) return e;
   }
   {
     StageTimer t(ST_SORT_PLACE, s);
-    const size_t lds = place_lds(a.n);
+    const size_t lds = place_lds(group_count(g, a.n));
     const auto kp = pick_aw<PlaceK>(a);
     int e = allow_lds(kp, lds);
     if (e) return e;
@@ -915,7 +942,13 @@ int scatter_run(Job& j, bool direct, const float* mesh_in, float* mesh_out, void
     e = check_hip(hipGetLastError(), "bucket place launch");
     if (e) return e;
   }
-  {
+  if (g.sort == SORT_PLANES) {
+    StageTimer t(ST_SCAN, s);
+    hipLaunchKernelGGL(k_plane_keys, dim3(a.n + 1), dim3(PKEY_NT), plane_keys_lds(g), s, j);
+    int e = check_hip(hipGetLastError(), "plane keys launch");
+    if (e) return e;
+  }
+  if (g.sort != SORT_KEYS) {
     StageTimer t(ST_SORT_FINE, s);
     const auto kf = a.stencil == PK_STENCIL_CIC_REF ? k_fine_place<PK_STENCIL_CIC_REF>
                     : a.stencil == PK_STENCIL_CIC   ? k_fine_place<PK_STENCIL_CIC>
@@ -969,22 +1002,28 @@ int scatter_sort_jobs(const Job* jobs, const BatchDims& d, hipStream_t s) {
   }
   {
     StageTimer t(ST_SCAN, s);
-    const int nb2 = (d.max_nkeys + SCAN_BLOCK - 1) / SCAN_BLOCK;
-    hipLaunchKernelGGL(k_col_scan_jobs, dim3((d.max_nkeys + COL_KEYS - 1) / COL_KEYS, nj), dim3(COL_NT), 0, s, jobs);
-    hipLaunchKernelGGL(k_scan_local_jobs, dim3(nb2, nj), dim3(SCAN_NT), 0, s, jobs);
-    hipLaunchKernelGGL(k_scan_add_jobs, dim3(nb2, nj), dim3(SCAN_NT), 0, s, jobs);
+    hipLaunchKernelGGL(k_columns_jobs, dim3(d.max_col, nj), dim3(COL_NT), 0, s, jobs);
     int e = check_hip(hipGetLastError(), "batch scan launch");
     if (e) return e;
   }
   {
     StageTimer t(ST_SORT_PLACE, s);
-    const size_t lds = place_lds(d.n);
+    // at least what any job's groups take (its rounds shrink as its groups grow)
+    const size_t lds = PLACE_LDS;
     int e = allow_lds(k_bucket_place_jobs, lds);
     if (e) return e;
     hipLaunchKernelGGL(k_bucket_place_jobs, dim3(d.max_nblk, nj), dim3(CNT_NT), lds, s, jobs);
     e = check_hip(hipGetLastError(), "batch bucket place launch");
     if (e) return e;
   }
+  if (d.planes) {
+    StageTimer t(ST_SCAN, s);
+    // at most 3 n / 2 keys per plane, whatever the job's tile
+    hipLaunchKernelGGL(k_plane_keys_jobs, dim3(d.n + 1, nj), dim3(PKEY_NT), (size_t)6 * d.n, s, jobs);
+    int e = check_hip(hipGetLastError(), "batch plane keys launch");
+    if (e) return e;
+  }
+  if (!d.fine) return PK_OK;
   StageTimer t(ST_SORT_FINE, s);
   int e = allow_lds(k_fine_place_jobs, FINE_LDS);
   if (e) return e;
