@@ -164,14 +164,13 @@ template <int M> __device__ __forceinline__ float2 tw_at(TwHalf<M> t, int q) {
 // COLFAST: consecutive threads take consecutive columns (else consecutive butterflies).
 // ------------------------------------------------------------------------------------
 template <int N, int R, int NS, int C, int PS, int CS, int NT, bool COLFAST, int TWS, int SK, class TW>
-__device__ __forceinline__ void fft_stage(float2* buf, TW tw) {
+__device__ __forceinline__ void fft_stage(float2* buf, TW tw, const int tid = threadIdx.x) {
   // point p of column c: p * PS + c * CS, plus p >> SK with a skew (SK > 0), which spreads
   // the stride-R autosort writes over the LDS banks
   auto at = [](int p, int c) { return p * PS + (SK > 0 ? (p >> SK) : 0) + c * CS; };
   constexpr int B = N / R;
   constexpr int TASKS = B * C;
   constexpr int PER = (TASKS + NT - 1) / NT;
-  const int tid = threadIdx.x;
   float2 v[PER][R];
 #pragma unroll
   for (int t = 0; t < PER; ++t) {
@@ -222,6 +221,108 @@ __device__ __forceinline__ void lds_fft(float2* buf, TW tw) {
   static_assert(SK == 0 || PS == 1, "skewed layouts take unit point stride");
   FFTStages<N, 0, 1, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw);
 }
+
+// ------------------------------------------------------------------------------------
+// Column transforms whose first stage takes its inputs from registers and whose last stage
+// leaves its outputs there.  Both touch rows j + r N / R of column c, for j = task / C and
+// c = task % C (task = threadIdx.x + t NT): the last stage's outputs of one transform are the
+// first stage's inputs of the next one, if that runs the radices in reverse (REV).  A
+// pointwise step between two transforms then costs no LDS round trip, and neither do the
+// loads and stores of a tile.  tid: the thread's index, made opaque once per tile
+// (opaque_tid): otherwise every address and twiddle index of the tile loop is computed once and
+// kept, and the registers spill.
+// ------------------------------------------------------------------------------------
+__device__ __forceinline__ int opaque_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+__host__ __device__ constexpr int radix_count(int N) {
+  int c = 0;
+  while (radix_at(N, c) > 1) ++c;
+  return c;
+}
+__host__ __device__ constexpr int plan_radix(int N, bool rev, int s) {
+  return radix_at(N, rev ? radix_count(N) - 1 - s : s);
+}
+__host__ __device__ constexpr int plan_ns(int N, bool rev, int s) {
+  int p = 1;
+  for (int i = 0; i < s; ++i) p *= plan_radix(N, rev, i);
+  return p;
+}
+
+template <int N, int C, int PS, int NT, bool REV> struct ColFFT {
+  static constexpr int L = radix_count(N);
+  static constexpr int R0 = plan_radix(N, REV, 0);
+  static constexpr int RL = plan_radix(N, REV, L - 1);
+  static constexpr int T0 = N / R0 * C, TL = N / RL * C;              // butterflies of the tile
+  static constexpr int PER0 = (T0 + NT - 1) / NT, PERL = (TL + NT - 1) / NT;
+
+  // f(t, r, row, column) for every input of this thread's first-stage butterflies
+  template <class F> static __device__ __forceinline__ void each_first(int tid, F&& f) {
+#pragma unroll
+    for (int t = 0; t < PER0; ++t) {
+      const int task = tid + t * NT;
+      if (T0 % NT == 0 || task < T0) {
+#pragma unroll
+        for (int r = 0; r < R0; ++r) f(t, r, task / C + r * (N / R0), task % C);
+      }
+    }
+  }
+  // f(t, r, row, column) for every output of this thread's last-stage butterflies
+  template <class F> static __device__ __forceinline__ void each_last(int tid, F&& f) {
+#pragma unroll
+    for (int t = 0; t < PERL; ++t) {
+      const int task = tid + t * NT;
+      if (TL % NT == 0 || task < TL) {
+#pragma unroll
+        for (int r = 0; r < RL; ++r) f(t, r, task / C + r * (N / RL), task % C);
+      }
+    }
+  }
+  // first stage: registers -> LDS.  The caller's barrier follows.  (A transform of one
+  // stage, N = 8, does it in last().)
+  static __device__ __forceinline__ void first(int tid, float2 (*v)[R0], float2* buf) {
+#pragma unroll
+    for (int t = 0; t < PER0; ++t) {
+      const int task = tid + t * NT;
+      if (T0 % NT == 0 || task < T0) {
+        if constexpr (L > 1) DFT<R0>::run(v[t]);
+#pragma unroll
+        for (int r = 0; r < R0; ++r) buf[(task / C * R0 + r) * PS + task % C] = v[t][r];
+      }
+    }
+  }
+  // the stages between, in LDS (they end with a barrier)
+  template <int S = 1, class TW> static __device__ __forceinline__ void middle(int tid, float2* buf, TW tw) {
+    if constexpr (S < L - 1) {
+      fft_stage<N, plan_radix(N, REV, S), plan_ns(N, REV, S), C, PS, 1, NT, true, 1, 0>(buf, tw, tid);
+      middle<S + 1>(tid, buf, tw);
+    }
+  }
+  // last stage: LDS -> registers.  A barrier must pass before the LDS is written again.
+  template <class TW> static __device__ __forceinline__ void last(int tid, const float2* buf, TW tw, float2 (*v)[RL]) {
+#pragma unroll
+    for (int t = 0; t < PERL; ++t) {
+      const int task = tid + t * NT;
+      if (TL % NT == 0 || task < TL) {
+        const int j = task / C;
+#pragma unroll
+        for (int r = 0; r < RL; ++r) v[t][r] = buf[(j + r * (N / RL)) * PS + task % C];
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < PERL; ++t) {
+      const int task = tid + t * NT;
+      if (TL % NT == 0 || task < TL) {
+        const int j = task / C;
+#pragma unroll
+        for (int r = 1; r < RL; ++r) v[t][r] = cmul(v[t][r], tw_at(tw, r * j));
+        DFT<RL>::run(v[t]);
+      }
+    }
+  }
+};
 
 // Copies an R x W block of complex values (global row stride gs, LDS row stride PS) into
 // LDS with every global load issued before the first LDS store, so each wave keeps all of

@@ -115,17 +115,63 @@ k_zpass(const float* __restrict__ mesh, float2* __restrict__ spec, const float2*
 // ------------------------------------------------------------------------------------
 // y pass: contiguous rows of N complex, in place
 // ------------------------------------------------------------------------------------
+// Which tiles (CY rows [kz][x] each) a pass takes, in what order, and what it stores.
+// Whole passes take the rows x-plane major from the highest x down: the z pass writes the rows
+// x-plane by x-plane upwards, so the first rows read here are the last it wrote (and an
+// inverse pass leaves the low x planes, which the C2R pass reads first, in the caches).  They
+// store the first half of their rows (the high x planes) non-temporally: the last-level
+// cache cannot hold the pass's output, and those rows would be evicted before the next pass
+// reads them, so they go to memory without displacing the second half (512^3: y pass 206 ->
+// 185 us, the next passes faster too; a quarter, three quarters or all of the rows
+// measured slower).
+template <int N> struct RowsWhole {
+  static constexpr int KZN = N / 2 + 1, XG = N / FFTCfg<N>::CY;
+  static constexpr int TILES = KZN * N / FFTCfg<N>::CY;
+  __device__ int tiles() const { return TILES; }
+  __device__ int tile(int t) const {
+    const int u = TILES - 1 - t;
+    return (u % KZN) * XG + u / KZN;
+  }
+  __device__ bool streamed(int t) const { return t < TILES / 2; }
+  __device__ bool keep(int) const { return true; }
+};
+// the rows of the lowest planes
+template <int N> struct RowsBelow {
+  int kz_lim;
+  __device__ int tiles() const { return (kz_lim + 1) * N / FFTCfg<N>::CY; }
+  __device__ int tile(int t) const { return t; }
+  __device__ bool streamed(int) const { return false; }
+  __device__ bool keep(int) const { return true; }
+};
+// the tiles that hold a row |x| <= R (separations, x and N - x alike), of which the columns
+// |y| <= R are stored
+template <int N> struct RowsNear {
+  static constexpr int C = FFTCfg<N>::CY, XG = N / C, KZN = N / 2 + 1;
+  int R, lo, cnt;   // per plane: the tiles [0, lo) and the last cnt - lo
+  __device__ explicit RowsNear(int R_) : R(R_) {
+    lo = min(R / C + 1, XG);
+    cnt = min(lo + (XG - (N - R) / C), XG);
+    if (R < 0) lo = cnt = 0;
+  }
+  __device__ int tiles() const { return cnt * KZN; }
+  __device__ int tile(int t) const {
+    const int u = tiles() - 1 - t, i = u / KZN;
+    return (u % KZN) * XG + (i < lo ? i : XG - cnt + i);
+  }
+  __device__ bool streamed(int) const { return false; }
+  __device__ bool keep(int y) const { return y <= R || N - y <= R; }
+};
+
 // CONJ: conj on load and store, i.e. the unnormalised inverse transform (e^{+i})
-// ntiles < 0: every tile; otherwise the first ntiles (rows [kz][x] of the lowest planes)
-template <int N, bool CONJ = false>
+template <int N, bool CONJ, class Rows>
 __device__ __forceinline__ void ypass_body(float2* __restrict__ spec, const float2* __restrict__ twg, int bx, int nbx,
-                                           int ntiles = -1) {
+                                           const Rows rows) {
   using Cf = FFTCfg<N>;
   // rows are skewed in LDS (point p at p + p / 8), which keeps the butterflies' strided
   // writes off each other's banks; twiddles from a quarter table
   constexpr int SK = 3;
   constexpr int C = Cf::CY, NT = Cf::NTY, CS = N + (SK > 0 ? (N >> SK) : 0) + 1;
-  const int NTILES = ntiles < 0 ? (N / 2 + 1) * N / C : ntiles;
+  const int NTILES = rows.tiles();
   __shared__ float2 buf[C * CS];
   __shared__ float2 twh[N / 2];
   const TwHalf<N> tw{twh};
@@ -146,35 +192,22 @@ __device__ __forceinline__ void ypass_body(float2* __restrict__ spec, const floa
       }
     }
   };
-  // Work item t -> tile.  Whole passes take the rows x-plane major from the highest x down:
-  // the z pass writes the rows x-plane by x-plane upwards, so the first rows read here are
-  // the last it wrote.
-  auto tile_of = [&](int t) -> int {
-    if (ntiles >= 0) return t;
-    constexpr int KZN = N / 2 + 1, XG = N / C;
-    const int u = NTILES - 1 - t;
-    return (u % KZN) * XG + u / KZN;
-  };
-  if (bx < NTILES) load(tile_of(bx));
+  if (bx < NTILES) load(rows.tile(bx));
   for (int item = bx; item < NTILES; item += nbx) {
-    const int tile = tile_of(item);
+    const int tile = rows.tile(item);
 #pragma unroll
     for (int k = 0; k < PER; ++k) {
       const int i = tid + k * NT;
       if (i < C * N) buf[at(i % N, i / N)] = pre[k];
     }
     __syncthreads();
-    if (item + nbx < NTILES) load(tile_of(item + nbx));
+    if (item + nbx < NTILES) load(rows.tile(item + nbx));
     lds_fft<N, C, 1, CS, NT, false, 1, SK>(buf, tw);
-    // Whole passes store the first half of their rows (the high x planes) non-temporally:
-    // the last-level cache cannot hold the pass's output, and those rows would be evicted
-    // before the x pass reads them, so they go to memory without displacing the second
-    // half (512^3: y pass 206 -> 185 us, the next passes faster too; a quarter, three
-    // quarters or all of the rows measured slower)
     float2* row = spec + (size_t)tile * C * N;
-    const bool streamed = ntiles < 0 && item < NTILES / 2;   // block-uniform
+    const bool streamed = rows.streamed(item);   // block-uniform
     typedef float f2v __attribute__((ext_vector_type(2)));
     for (int i = tid; i < C * N; i += NT) {
+      if (!rows.keep(i % N)) continue;
       float2 v = buf[at(i % N, i / N)];
       if constexpr (CONJ) v.y = -v.y;
       if (streamed) {
@@ -226,7 +259,7 @@ __device__ __forceinline__ void mass_finalize_block(const Job& j) {
 
 template <int N>
 __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass(float2* __restrict__ spec, const float2* __restrict__ twg) {
-  ypass_body<N>(spec, twg, blockIdx.x, gridDim.x);
+  ypass_body<N, false>(spec, twg, blockIdx.x, gridDim.x, RowsWhole<N>());
 }
 
 // y pass of a fused estimate whose last block first does the mass finalize (the last block
@@ -234,13 +267,13 @@ __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass(float2* __restrict__ s
 template <int N>
 __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_mass(Job j, const float2* __restrict__ twg) {
   if (blockIdx.x == gridDim.x - 1) mass_finalize_block<FFTCfg<N>::NTY>(j);
-  ypass_body<N>(j.spec, twg, blockIdx.x, gridDim.x);
+  ypass_body<N, false>(j.spec, twg, blockIdx.x, gridDim.x, RowsWhole<N>());
 }
 
 template <int N>
 __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_lim(float2* __restrict__ spec,
                                                               const float2* __restrict__ twg, int kz_lim) {
-  ypass_body<N>(spec, twg, blockIdx.x, gridDim.x, (kz_lim + 1) * N / FFTCfg<N>::CY);
+  ypass_body<N, false>(spec, twg, blockIdx.x, gridDim.x, RowsBelow<N>{kz_lim});
 }
 
 template <int N>
@@ -249,7 +282,7 @@ __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_jobs(const Job* __rest
   const Job& j = jobs[blockIdx.y];
   if (!j.active) return;
   if (blockIdx.x == gridDim.x - 1) mass_finalize_block<FFTCfg<N>::NTY>(j);   // fused jobs
-  ypass_body<N>(j.spec, twg, blockIdx.x, gridDim.x);
+  ypass_body<N, false>(j.spec, twg, blockIdx.x, gridDim.x, RowsWhole<N>());
 }
 
 // ------------------------------------------------------------------------------------
@@ -884,11 +917,17 @@ k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__
   }
 }
 
-// kz_lim: planes above it are not transformed (they are zero for the caller)
 template <int N>
 __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_inverse(float2* __restrict__ spec,
-                                                                  const float2* __restrict__ twg, int kz_lim) {
-  ypass_body<N, true>(spec, twg, blockIdx.x, gridDim.x, (kz_lim + 1) * N / FFTCfg<N>::CY);
+                                                                  const float2* __restrict__ twg) {
+  ypass_body<N, true>(spec, twg, blockIdx.x, gridDim.x, RowsWhole<N>());
+}
+
+// kz_lim: planes above it are not transformed (they are zero for the caller)
+template <int N>
+__global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_inverse_lim(float2* __restrict__ spec,
+                                                                      const float2* __restrict__ twg, int kz_lim) {
+  ypass_body<N, true>(spec, twg, blockIdx.x, gridDim.x, RowsBelow<N>{kz_lim});
 }
 
 // Half-spectrum rows B[kz][x][y] (kz = 0..N/2, transformed in x and y) -> real rows
@@ -1189,54 +1228,106 @@ __global__ void __launch_bounds__(64) k_bispec_bq(BispecArgs a, int n) {
 //   x pass: forward DFT along x, |delta_k|^2 W_k times irfftn's 1/n^3 (2/n^3 on interior
 //           kz planes), inverse DFT along kx; FP64 partials of their sum = xi(s = 0),
 //           the largest value of the separation grid (|xi(s)| <= xi(0) for a spectrum >= 0)
-//   y pass: inverse (k_ypass_inverse)
+//   y pass: inverse (k_ypass_inverse_near)
 //   z pass: C2R rows binned by |s| on the fly (the n^3 separation grid is never stored):
 //           each thread walks a run of z, sums in FP64 while the bin stays the same and
 //           adds each run to 64-bit fixed-point LDS bins (integer sums do not depend on
 //           order, so results are run-to-run identical); blocks add their bins to global
 //           accumulators; S = 2^e with (n^3 2 xi(0)) S < 2^62 bounds every bin sum
 // ------------------------------------------------------------------------------------
+// Separations beyond the last bin's end need no values: with R = floor(sqrt(thr[nb] - 1)), a
+// row (x, y) of the grid holds a binned cell only if |x|, |y| <= R.  The x pass stores, and the
+// passes after it transform, those rows alone.  s <= 200 Mpc/h in a 1500 Mpc/h box at 512^3
+// (27% of the x planes, 7% of the rows): inverse y pass 219 -> 59 us, C2R and binning 337 -> 74.
+// thr is read on the device: a caller holds it there only.
+__device__ __forceinline__ int xi_radius(const XiArgs& a, int n) {
+  const int e = a.thr[a.nb];
+  if (e <= 0) return -1;
+  int r = (int)sqrtf((float)(e - 1));
+  if (r * r > e - 1) --r;
+  else if ((r + 1) * (r + 1) <= e - 1) ++r;
+  return min(r, n / 2);
+}
+
+// LDS: the tile, half the twiddles, the window row; blocks per CU and the register budget
+template <int N> struct XPowerCfg {
+  static constexpr int C = FFTCfg<N>::CX, NT = FFTCfg<N>::NTX;
+  static constexpr size_t LDS = (size_t)N * (C + 1) * 8 + (size_t)N / 2 * 8 + (size_t)N * 4 + (NT / 64 + 1) * 8;
+  static constexpr int WPE = N < 64 ? 1 : cmax(1, cmin(4, (int)((160 * 1024) / LDS) * (NT / 64) / 4));
+};
+
+// Bound by LDS traffic and FFT instructions.  The power is taken in registers between the
+// forward transform's last stage and the inverse's first, the tile is loaded and stored from
+// registers, and rows beyond the radius are not stored: 342 -> 217 us at 512^3 (39 bins to
+// 200 Mpc/h in a 1500 Mpc/h box; 234 us with every row stored).
 template <int N>
-__global__ void __launch_bounds__(FFTCfg<N>::NTX)
+__global__ void __launch_bounds__(FFTCfg<N>::NTX) __attribute__((amdgpu_waves_per_eu(XPowerCfg<N>::WPE)))
 k_xpass_power_inverse(float2* __restrict__ spec, const float2* __restrict__ twg, const float* __restrict__ wt,
-                      double* __restrict__ xi0_part) {
+                      XiArgs a) {
   using Cf = FFTCfg<N>;
   constexpr int C = Cf::CX, NT = Cf::NTX, PS = C + 1;
   constexpr int YT = N / C;
   constexpr int NTILES = (N / 2 + 1) * YT;
   constexpr int H = N / 2;
+  using F = ColFFT<N, C, PS, NT, false>;
+  using B = ColFFT<N, C, PS, NT, true>;
   __shared__ float2 buf[N * PS];
-  __shared__ float2 tw[N];
-  __shared__ double red[NT];
+  __shared__ float2 twh[N / 2];
+  __shared__ float wt_s[N];
+  __shared__ double red[NT / 64 + 1];
+  const TwHalf<N> tw{twh};
   const int tid = threadIdx.x;
-  for (int i = tid; i < N; i += NT) tw[i] = twg[i];
+  for (int i = tid; i < N / 2; i += NT) twh[i] = twg[i];
+  for (int i = tid; i < N; i += NT) wt_s[i] = wt[i];
+  const int R = xi_radius(a, N);
   const double s_edge = 1.0 / ((double)N * (double)N * (double)N);
   double acc = 0.0;
+  __syncthreads();
   for (int tile = blockIdx.x; tile < NTILES; tile += gridDim.x) {
     const int kz = tile / YT, yt = tile % YT;
     const float sc = (float)((kz == 0 || kz == H) ? s_edge : 2.0 * s_edge);
     float2* base = spec + (size_t)kz * N * N + (size_t)yt * C;
-    stage_tile<N, C, PS, NT>(buf, base, N);
-    __syncthreads();
-    lds_fft<N, C, PS, 1, NT, true, 1>(buf, tw);
-    const float wz = wt[kz];
-    for (int i = tid; i < N * C; i += NT) {
-      const int c = i % C, r = i / C;
-      const float2 v = buf[r * PS + c];
-      const float pw = (v.x * v.x + v.y * v.y) * (wt[r] * wt[yt * C + c] * wz) * sc;
-      acc += (double)pw;
-      buf[r * PS + c] = make_float2(pw, 0.0f);   // real: its conjugate is itself
+    const int to = opaque_tid();
+    {
+      float2 v[F::PER0][F::R0];
+      F::each_first(to, [&](int t, int r, int row, int c) { v[t][r] = base[row * N + c]; });
+      F::first(to, v, buf);
     }
     __syncthreads();
-    lds_fft<N, C, PS, 1, NT, true, 1>(buf, tw);
-    for (int i = tid; i < N * C; i += NT) {
-      const float2 v = buf[(i / C) * PS + (i % C)];
-      base[(size_t)(i / C) * N + (i % C)] = make_float2(v.x, -v.y);
+    F::middle(to, buf, tw);
+    {
+      float2 v[F::PERL][F::RL];
+      F::last(to, buf, tw, v);
+      const float wz = wt_s[kz];
+      F::each_last(to, [&](int t, int r, int row, int c) {
+        const float2 x = v[t][r];
+        const float pw = (x.x * x.x + x.y * x.y) * (wt_s[row] * wt_s[yt * C + c] * wz) * sc;
+        acc += (double)pw;
+        v[t][r] = make_float2(pw, 0.0f);   // real: its conjugate is itself
+      });
+      __syncthreads();   // every row read before the inverse's first stage overwrites them
+      B::first(to, v, buf);
     }
     __syncthreads();
+    B::middle(to, buf, tw);
+    {
+      float2 v[B::PERL][B::RL];
+      B::last(to, buf, tw, v);
+      B::each_last(to, [&](int t, int r, int row, int c) {
+        if (row <= R || N - row <= R) base[row * N + c] = make_float2(v[t][r].x, -v[t][r].y);
+      });
+    }
+    __syncthreads();   // the tile is read before the next one's first stage overwrites it
   }
-  const double t = block_sum_f64(acc, red, NT);
-  if (tid == 0) xi0_part[blockIdx.x] = t;
+  const double t = block_sum_f64_waves<NT>(acc, red);
+  if (tid == 0) a.xi0_part[blockIdx.x] = t;
+}
+
+// inverse y pass of the rows that hold a binned separation
+template <int N>
+__global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_inverse_near(float2* __restrict__ spec,
+                                                                       const float2* __restrict__ twg, XiArgs a) {
+  ypass_body<N, true>(spec, twg, blockIdx.x, gridDim.x, RowsNear<N>(xi_radius(a, N)));
 }
 
 // fixed-order xi(0) -> scale; clears the accumulators of this estimate
@@ -1276,7 +1367,6 @@ k_zpass_c2r_bin(const float2* __restrict__ bspec, const float2* __restrict__ twg
   using BC = XiBinCfg<N>;
   constexpr int NC = Cf::NC, C = Cf::CZ, NT = Cf::NTZ, CS = NC + 1;
   constexpr int YT = N / C;
-  constexpr int NTILES = N * YT;
   constexpr int H = N / 2;
   constexpr int CH = BC::CH;
   __shared__ float2 buf[C * CS];
@@ -1291,8 +1381,14 @@ k_zpass_c2r_bin(const float2* __restrict__ bspec, const float2* __restrict__ twg
   for (int i = tid; i <= nb; i += NT) thr_s[i] = a.thr[i];
   for (int i = tid; i < a.jlen; i += NT) jst_s[i] = a.jst[i];
   const double S = a.scale[0];
-  for (int tile = blockIdx.x; tile < NTILES; tile += gridDim.x) {
-    const int x = tile / YT, yt = tile % YT;
+  // the planes |x| <= R and the row tiles that hold a row |y| <= R (the other rows of such a
+  // tile hold no binned cell and whatever the spectrum held: their runs are skipped below)
+  const int R = xi_radius(a, N);
+  const int nx = R < 0 ? 0 : min(2 * R + 1, N);
+  const int ylo = min(R / C + 1, YT), ny = min(ylo + (YT - (N - R) / C), YT);
+  for (int item = blockIdx.x; item < nx * ny; item += gridDim.x) {
+    const int ix = item / ny, iy = item % ny;
+    const int x = ix <= R ? ix : N - nx + ix, yt = iy < ylo ? iy : YT - ny + iy;
     {
       constexpr int TOT = (NC + 1) * C, PER = (TOT + NT - 1) / NT;
       float2 v[PER];
@@ -1597,7 +1693,7 @@ template <int N> struct FFTLaunch {
     if (!gz) gz = persistent_grid(k_zpass_c2r<N>, Cf::NTZ, ZTILES);
     StageTimer t(ST_ADJOINT_FFT, s);
     hipLaunchKernelGGL(k_xpass_adjoint<N>, dim3(gx), dim3(Cf::NTX), 0, s, j, tw, coef, bspec);
-    hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, bspec, tw, N / 2);
+    hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, bspec, tw);
     hipLaunchKernelGGL(k_zpass_c2r<N>, dim3(gz), dim3(Cf::NTZ), 0, s, (const float2*)bspec, tw, gmesh, N / 2);
     return check_hip(hipGetLastError(), "adjoint FFT launch");
   }
@@ -1634,13 +1730,13 @@ template <int N> struct FFTLaunch {
   static int shell_inverse(bool one, const float2* spec, float2* scratch, const float2* tw, ShellMask sm,
                            hipStream_t s) {
     static int gy = 0;
-    if (!gy) gy = persistent_grid(k_ypass_inverse<N>, Cf::NTY, YTILES);
+    if (!gy) gy = persistent_grid(k_ypass_inverse_lim<N>, Cf::NTY, YTILES);
     FieldGen g{};
     g.n = N;
     const int kl = shell_kz_lim(sm.hi);
     int e = one ? xinv<C2R_SHELL_ONE>(spec, scratch, tw, g, s, sm, kl) : xinv<C2R_SHELL>(spec, scratch, tw, g, s, sm, kl);
     if (e) return e;
-    if (kl >= 0) hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, scratch, tw, kl);
+    if (kl >= 0) hipLaunchKernelGGL(k_ypass_inverse_lim<N>, dim3(gy), dim3(Cf::NTY), 0, s, scratch, tw, kl);
     return check_hip(hipGetLastError(), "shell inverse launch");
   }
   // forward transform of the planes kz <= kz_lim only (higher planes are left unwritten)
@@ -1715,7 +1811,7 @@ template <int N> struct FFTLaunch {
             : src == C2R_DELTA  ? xinv<C2R_DELTA>(in, scratch, tw, g, s)
                                 : xinv<C2R_PSI_Z>(in, scratch, tw, g, s);
     if (e) return e;
-    hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, scratch, tw, N / 2);
+    hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, scratch, tw);
     hipLaunchKernelGGL(k_zpass_c2r<N>, dim3(gz), dim3(Cf::NTZ), 0, s, (const float2*)scratch, tw, mesh, N / 2);
     return check_hip(hipGetLastError(), "inverse FFT launch");
   }
@@ -1727,14 +1823,14 @@ template <int N> struct FFTLaunch {
   static int xi(const float* mesh, float2* spec, const float2* tw, const float* wt, const XiArgs& a,
                 hipStream_t s) {
     static int gy = 0, gz = 0;
-    if (!gy) gy = persistent_grid(k_ypass_inverse<N>, Cf::NTY, YTILES);
+    if (!gy) gy = persistent_grid(k_ypass_inverse_near<N>, Cf::NTY, YTILES);
     if (!gz) gz = persistent_grid(k_zpass_c2r_bin<N>, Cf::NTZ, ZTILES);   // sized without dynamic LDS
     int e = zpass(mesh, spec, tw, nullptr, nullptr, nullptr, s);
     if (!e) e = ypass(spec, tw, s);
     if (e) return e;
-    hipLaunchKernelGGL(k_xpass_power_inverse<N>, dim3(xi_gx()), dim3(Cf::NTX), 0, s, spec, tw, wt, a.xi0_part);
+    hipLaunchKernelGGL(k_xpass_power_inverse<N>, dim3(xi_gx()), dim3(Cf::NTX), 0, s, spec, tw, wt, a);
     hipLaunchKernelGGL(k_xi_scale, dim3(1), dim3(256), 0, s, a, N);
-    hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, spec, tw, N / 2);
+    hipLaunchKernelGGL(k_ypass_inverse_near<N>, dim3(gy), dim3(Cf::NTY), 0, s, spec, tw, a);
     hipLaunchKernelGGL(k_zpass_c2r_bin<N>, dim3(gz), dim3(Cf::NTZ), (size_t)a.nb * 3 * sizeof(unsigned long long), s,
                        (const float2*)spec, tw, a);
     hipLaunchKernelGGL(k_xi_finalize, dim3((a.nb + 255) / 256), dim3(256), 0, s, a, N);
