@@ -41,8 +41,9 @@ template <int N, int TY_> struct FusedCfg {
   // blocks of this tile size a CU holds; with two or more, 512 threads each (registers)
   static constexpr int BPC = (int)((160 * 1024) / (LDS + STATIC_LDS));
   // at least 512 threads: small meshes have dense tiles, and the deposit of their records
-  // needs the parallelism even where the z transform alone would use fewer threads
-  static constexpr int NT0 = cmin(1024, cmax(cmin(512, TY * N), (TY * NC / 8) / 64 * 64));
+  // needs the parallelism even where the z transform alone would use fewer threads.  Whole
+  // waves: the mass and square sums go by wave.
+  static constexpr int NT0 = cmin(1024, cmax(cmin(512, (TY * N + 63) / 64 * 64), (TY * NC / 8) / 64 * 64));
   static constexpr int NT = BPC >= 2 ? cmin(NT0, 512) : NT0;
   static constexpr int PER = (TY * N + NT - 1) / NT;     // cells per thread in the conversion
   // waves per SIMD the LDS allows (capped at 4): the register budget is held to it
