@@ -516,12 +516,13 @@ struct BackwardWS {
   float2* bspec;
   float* gmesh;
   float* coef;
-  void* gather;
-  size_t gather_bytes;
+  double* gsum_part;   // [parts]
+  int parts;
+  double* gbar;
   size_t bytes;
 };
 
-BackwardWS carve_backward(int n, int64_t np, int nb, void* base) {
+BackwardWS carve_backward(int n, int nb, void* base) {
   BackwardWS w{};
   char* b = static_cast<char*>(base);
   size_t off = 0;
@@ -533,8 +534,9 @@ BackwardWS carve_backward(int n, int64_t np, int nb, void* base) {
   w.bspec = static_cast<float2*>(take((size_t)(n / 2 + 1) * n * n * sizeof(float2)));
   w.gmesh = static_cast<float*>(take((size_t)n * n * n * sizeof(float)));
   w.coef = static_cast<float*>(take((size_t)nb * 3 * sizeof(float)));
-  w.gather_bytes = gather_workspace_bytes(np);
-  w.gather = take(w.gather_bytes);
+  w.parts = fft_adjoint_grid(n, nb);
+  w.gsum_part = static_cast<double*>(take((size_t)w.parts * sizeof(double)));
+  w.gbar = static_cast<double*>(take(sizeof(double)));
   w.bytes = off;
   return w;
 }
@@ -546,7 +548,7 @@ int pk_estimate_backward_workspace_size(pk_plan* p, int64_t np, int nb, size_t* 
   if (!bytes) return set_error(PK_E_INVALID, "null bytes pointer");
   if (nb < 1) return set_error(PK_E_INVALID, "need at least one bin (nb=%d)", nb);
   if (np < 0 || np > 0x7fffffffLL) return set_error(PK_E_INVALID, "particle count out of range");
-  *bytes = carve_backward(p->n, np, nb, nullptr).bytes;
+  *bytes = carve_backward(p->n, nb, nullptr).bytes;
   return PK_OK;
 }
 
@@ -573,7 +575,7 @@ int pk_estimate_backward(pk_plan* p, const float* x, int64_t sx, const float* y,
   if (e) return e;
   if (fwd_workspace_bytes < fw.bytes)
     return set_error(PK_E_WORKSPACE, "forward workspace %zu < %zu bytes", fwd_workspace_bytes, fw.bytes);
-  BackwardWS bw = carve_backward(p->n, np, nb, workspace);
+  BackwardWS bw = carve_backward(p->n, nb, workspace);
   if (workspace_bytes < bw.bytes)
     return set_error(PK_E_WORKSPACE, "backward workspace %zu < %zu bytes", workspace_bytes, bw.bytes);
   hipStream_t s = as_stream(stream);
@@ -586,9 +588,9 @@ int pk_estimate_backward(pk_plan* p, const float* x, int64_t sx, const float* y,
   set_bin_fields(j, p, fw.spec, thr, jstart, counts, nullptr, nb, window_p, PK_FLAG_ZERO_DC, box_size, 0.0, nullptr,
                  nullptr, nullptr, nullptr, nullptr);
   j.scale_stats = fw.fused ? stats : nullptr;   // fused: the spectrum is of rho - c, delta_k = S spec_k
-  e = fft_adjoint(n, j, p->tw, bw.coef, bw.bspec, bw.gmesh, s);
+  e = fft_adjoint(n, j, p->tw, bw.coef, bw.bspec, bw.gmesh, bw.gsum_part, s);
   if (e) return e;
-  return gather_gradients(a, bw.gmesh, stats, grad_pos, grad_w, bw.gather, bw.gather_bytes, s);
+  return gather_gradients(a, bw.gmesh, stats, bw.gsum_part, bw.parts, bw.gbar, grad_pos, grad_w, s);
 }
 
 // ------------------------------------------------------------------------------------

@@ -862,59 +862,122 @@ __global__ void __launch_bounds__(FIN_NT) k_bin_finalize_jobs(const Job* __restr
 // Three passes mirror the forward ones: x (forward FFT, times 2 G S, inverse FFT),
 // y (inverse), z (half-spectrum to real rows).
 // ------------------------------------------------------------------------------------
-template <int N>
-__global__ void __launch_bounds__(FFTCfg<N>::NTX)
-k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__ coef, float2* __restrict__ bspec) {
+// The x pass also sums 2 G_k |delta_k|^2 = Re A_k conj(delta_k) over the stored modes: by Parseval,
+// with A_0 = 0, that is n^3 gbar, gbar = sum_x g(x) rho(x) / M (the mean density's dependence on
+// the particles), which would otherwise take a pass of scattered reads over them (143 us for 2e6
+// particles at 256^3).
+// Tile and inverse as in the xi x pass: the factor is applied in registers between the forward
+// transform's last stage and the inverse's first (417 -> 382 us at 512^3; bound by the factors'
+// arithmetic).
+// LH: bin tables and coefficients in LDS (nb <= HB_LDS)
+template <int N> struct XAdjCfg {
+  static constexpr int C = FFTCfg<N>::CX, NT = FFTCfg<N>::NTX;
+  static constexpr int JLEN = isqrt_c(3 * (N / 2) * (N / 2)) + 2;
+  static constexpr size_t LDS = (size_t)N * (C + 1) * 8 + (size_t)N / 2 * 8 + (size_t)N * 4 + (NT / 64 + 1) * 8 +
+                                (size_t)JLEN * 2 + (HB_LDS + 1) * 4 + 3 * HB_LDS * 4;
+  static constexpr int WPE = N < 64 ? 1 : cmax(1, cmin(4, (int)((160 * 1024) / LDS) * (NT / 64) / 4));
+};
+template <int N, bool LH>
+__global__ void __launch_bounds__(FFTCfg<N>::NTX) __attribute__((amdgpu_waves_per_eu(XAdjCfg<N>::WPE)))
+k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__ coef_g, float2* __restrict__ bspec,
+                double* __restrict__ gsum_part) {
   using Cf = FFTCfg<N>;
   constexpr int C = Cf::CX, NT = Cf::NTX, PS = C + 1;
   constexpr int YT = N / C;
   constexpr int NTILES = (N / 2 + 1) * YT;
   constexpr int H = N / 2;
+  constexpr int JLEN = XAdjCfg<N>::JLEN;
+  using F = ColFFT<N, C, PS, NT, false>;
+  using B = ColFFT<N, C, PS, NT, true>;
   __shared__ float2 buf[N * PS];
+  __shared__ float2 twh[N / 2];
+  __shared__ float wt[N];
+  __shared__ double red[NT / 64 + 1];
+  __shared__ int thr_s[LH ? HB_LDS + 1 : 1];
+  __shared__ short jst_s[LH ? JLEN : 1];
+  __shared__ float coef_s[LH ? 3 * HB_LDS : 1];
+  const TwHalf<N> tw{twh};
   const float2* __restrict__ spec = j.spec;
-  const float* __restrict__ wt = j.wtab;
-  const int* __restrict__ thr = j.thr;
-  const int* __restrict__ jst = j.jst;
   const int nb = j.nb;
   const float sf = j.scale_stats ? (float)j.scale_stats[1] : 1.0f;
   const int tid = threadIdx.x;
+  for (int i = tid; i < N / 2; i += NT) twh[i] = twg[i];
+  for (int i = tid; i < N; i += NT) wt[i] = j.wtab[i];
+  if constexpr (LH) {
+    for (int i = tid; i <= nb; i += NT) thr_s[i] = j.thr[i];
+    for (int i = tid; i < JLEN; i += NT) jst_s[i] = (short)j.jst[i];
+    for (int i = tid; i < 3 * nb; i += NT) coef_s[i] = coef_g[i];
+  }
+  auto slot_of = [&](int m) -> int {
+    if constexpr (LH) return find_bin(m, thr_s, jst_s, nb);
+    else return find_bin(m, j.thr, j.jst, nb);
+  };
+  auto coef = [&](int i) -> float {
+    if constexpr (LH) return coef_s[i];
+    else return coef_g[i];
+  };
+  double acc = 0.0;
+  __syncthreads();
   for (int tile = blockIdx.x; tile < NTILES; tile += gridDim.x) {
     const int kz = tile / YT, yt = tile % YT;
-    stage_tile<N, C, PS, NT>(buf, spec + (size_t)kz * N * N + (size_t)yt * C, N);
-    __syncthreads();
-    lds_fft<N, C, PS, 1, NT, true, 1>(buf, twg);
-    const float wz = wt[kz];
-    const int kz2 = kz * kz;
-    for (int i = tid; i < N * C; i += NT) {
-      const int c = i % C, r = i / C;
-      const int y = yt * C + c;
-      const int kx = r <= H ? r : r - N;
-      const int ky = y <= H ? y : y - N;
-      const int m = kx * kx + ky * ky + kz2;
-      float g = 0.0f;
-      if (m > 0) {   // the k = 0 mode is exactly 0 in the forward (contrast applied)
-        const int slot = find_bin(m, thr, jst, nb);
-        if (slot >= 0) {
-          const float rm = 1.0f / (float)m;
-          const float l2 = 0.5f * (float)(3 * kz2 - m) * rm;
-          const double num4 = (double)kz2 * (35.0 * (double)kz2 - 30.0 * (double)m) + 3.0 * (double)m * (double)m;
-          const float l4 = 0.125f * (float)num4 * rm * rm;
-          g = wt[r] * wt[y] * wz * (coef[3 * slot] + coef[3 * slot + 1] * l2 + coef[3 * slot + 2] * l4);
-        }
-      }
-      const float sc = 2.0f * g * sf;
-      const float2 v = buf[r * PS + c];
-      buf[r * PS + c] = make_float2(sc * v.x, -sc * v.y);   // conj(A): inverse via the forward FFT
-    }
-    __syncthreads();
-    lds_fft<N, C, PS, 1, NT, true, 1>(buf, twg);
+    const float2* base = spec + (size_t)kz * N * N + (size_t)yt * C;
     float2* ob = bspec + (size_t)kz * N * N + (size_t)yt * C;
-    for (int i = tid; i < N * C; i += NT) {
-      const float2 v = buf[(i / C) * PS + (i % C)];
-      ob[(size_t)(i / C) * N + (i % C)] = make_float2(v.x, -v.y);
+    const int to = opaque_tid();
+    {
+      float2 v[F::PER0][F::R0];
+      F::each_first(to, [&](int t, int r, int row, int c) { v[t][r] = base[row * N + c]; });
+      F::first(to, v, buf);
+    }
+    // the factors of the modes this thread will hold, while no transform values occupy its
+    // registers (computed after the last stage, they spill)
+    float sc[F::PERL][F::RL];
+    {
+      const float wz = wt[kz];
+      const int kz2 = kz * kz;
+      F::each_last(to, [&](int t, int r, int row, int c) {
+        const int y = yt * C + c;
+        const int kx = row <= H ? row : row - N;
+        const int ky = y <= H ? y : y - N;
+        const int m = kx * kx + ky * ky + kz2;
+        float g = 0.0f;
+        if (m > 0) {   // the k = 0 mode is exactly 0 in the forward (contrast applied)
+          const int slot = slot_of(m);
+          if (slot >= 0) {
+            const float rm = 1.0f / (float)m;
+            const float l2 = 0.5f * (float)(3 * kz2 - m) * rm;
+            const double num4 = (double)kz2 * (35.0 * (double)kz2 - 30.0 * (double)m) + 3.0 * (double)m * (double)m;
+            const float l4 = 0.125f * (float)num4 * rm * rm;
+            g = wt[row] * wt[y] * wz * (coef(3 * slot) + coef(3 * slot + 1) * l2 + coef(3 * slot + 2) * l4);
+          }
+        }
+        sc[t][r] = 2.0f * g * sf;
+        __builtin_amdgcn_sched_barrier(0);
+      });
     }
     __syncthreads();
+    F::middle(to, buf, tw);
+    {
+      float2 v[F::PERL][F::RL];
+      F::last(to, buf, tw, v);
+      F::each_last(to, [&](int t, int r, int, int) {
+        const float2 d = v[t][r];
+        acc += (double)(sc[t][r] * (d.x * d.x + d.y * d.y));
+        v[t][r] = make_float2(sc[t][r] * d.x, -sc[t][r] * d.y);   // conj(A): inverse via the forward FFT
+      });
+      __syncthreads();   // every row read before the inverse's first stage overwrites them
+      B::first(to, v, buf);
+    }
+    __syncthreads();
+    B::middle(to, buf, tw);
+    {
+      float2 v[B::PERL][B::RL];
+      B::last(to, buf, tw, v);
+      B::each_last(to, [&](int t, int r, int row, int c) { ob[row * N + c] = make_float2(v[t][r].x, -v[t][r].y); });
+    }
+    __syncthreads();   // the tile is read before the next one's first stage overwrites it
   }
+  const double t = block_sum_f64_waves<NT>(acc * (double)sf, red);
+  if (tid == 0) gsum_part[blockIdx.x] = t;
 }
 
 template <int N>
@@ -936,7 +999,8 @@ __global__ void __launch_bounds__(FFTCfg<N>::NTY) k_ypass_inverse_lim(float2* __
 // inverse FFT of Z_k = (Y_k + conj Y_{N/2-k}) + i e^{2 pi i k / N} (Y_k - conj Y_{N/2-k}),
 // whose outputs are u(2j) + i u(2j+1).
 // planes kz > kz_lim are taken as zero (not read)
-template <int N>
+// BRICK: out is in bricks of 2 x 4 x 4 cells, one 128-byte line each (brick_index)
+template <int N, bool BRICK = false>
 __global__ void __launch_bounds__(FFTCfg<N>::NTZ)
 k_zpass_c2r(const float2* __restrict__ bspec, const float2* __restrict__ twg, float* __restrict__ out, int kz_lim) {
   using Cf = FFTCfg<N>;
@@ -993,11 +1057,21 @@ k_zpass_c2r(const float2* __restrict__ bspec, const float2* __restrict__ twg, fl
     }
     __syncthreads();
     lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw);
-    float2* orow = reinterpret_cast<float2*>(out + ((size_t)x * N + (size_t)yt * C) * N);
-    for (int i = tid; i < C * NC; i += NT) {
-      const int c = i / NC, jj = i % NC;
-      const float2 v = buf[c * CS + jj];
-      orow[(size_t)c * NC + jj] = make_float2(v.x, -v.y);   // (u(2j), u(2j+1))
+    if constexpr (BRICK) {
+      // four z of one row per lane, four rows of a brick per 64 bytes
+      static_assert(C % 4 == 0 && NC % 2 == 0, "whole brick rows");
+      for (int i = tid; i < C * NC / 2; i += NT) {
+        const int c = (i & 3) + 4 * (i / (2 * NC)), q = (i >> 2) % (NC / 2);
+        const float2 a = buf[c * CS + 2 * q], b = buf[c * CS + 2 * q + 1];
+        *reinterpret_cast<float4*>(out + brick_index(N, x, yt * C + c, 4 * q)) = make_float4(a.x, -a.y, b.x, -b.y);
+      }
+    } else {
+      float2* orow = reinterpret_cast<float2*>(out + ((size_t)x * N + (size_t)yt * C) * N);
+      for (int i = tid; i < C * NC; i += NT) {
+        const int c = i / NC, jj = i % NC;
+        const float2 v = buf[c * CS + jj];
+        orow[(size_t)c * NC + jj] = make_float2(v.x, -v.y);   // (u(2j), u(2j+1))
+      }
     }
     __syncthreads();
   }
@@ -1686,15 +1760,28 @@ template <int N> struct FFTLaunch {
     }
     return e ? e : check_hip(hipGetLastError(), "x pass + bin launch");
   }
-  static int adjoint(const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh, hipStream_t s) {
-    static int gx = 0, gy = 0, gz = 0;
-    if (!gx) gx = persistent_grid(k_xpass_adjoint<N>, Cf::NTX, XTILES);
+  static int adjoint_grid(bool lh) {
+    static int g_l = 0, g_g = 0;
+    int& g = lh ? g_l : g_g;
+    if (!g) g = lh ? persistent_grid(k_xpass_adjoint<N, true>, Cf::NTX, XTILES)
+                   : persistent_grid(k_xpass_adjoint<N, false>, Cf::NTX, XTILES);
+    return g;
+  }
+  static int adjoint(const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh,
+                     double* gsum_part, hipStream_t s) {
+    static int gy = 0, gz = 0;
     if (!gy) gy = persistent_grid(k_ypass_inverse<N>, Cf::NTY, YTILES);
-    if (!gz) gz = persistent_grid(k_zpass_c2r<N>, Cf::NTZ, ZTILES);
+    if (!gz) gz = persistent_grid(k_zpass_c2r<N, true>, Cf::NTZ, ZTILES);
+    const bool lh = j.nb <= HB_LDS;
     StageTimer t(ST_ADJOINT_FFT, s);
-    hipLaunchKernelGGL(k_xpass_adjoint<N>, dim3(gx), dim3(Cf::NTX), 0, s, j, tw, coef, bspec);
+    if (lh)
+      hipLaunchKernelGGL((k_xpass_adjoint<N, true>), dim3(adjoint_grid(true)), dim3(Cf::NTX), 0, s, j, tw, coef,
+                         bspec, gsum_part);
+    else
+      hipLaunchKernelGGL((k_xpass_adjoint<N, false>), dim3(adjoint_grid(false)), dim3(Cf::NTX), 0, s, j, tw, coef,
+                         bspec, gsum_part);
     hipLaunchKernelGGL(k_ypass_inverse<N>, dim3(gy), dim3(Cf::NTY), 0, s, bspec, tw);
-    hipLaunchKernelGGL(k_zpass_c2r<N>, dim3(gz), dim3(Cf::NTZ), 0, s, (const float2*)bspec, tw, gmesh, N / 2);
+    hipLaunchKernelGGL((k_zpass_c2r<N, true>), dim3(gz), dim3(Cf::NTZ), 0, s, (const float2*)bspec, tw, gmesh, N / 2);
     return check_hip(hipGetLastError(), "adjoint FFT launch");
   }
   template <int SRC>
@@ -1983,9 +2070,19 @@ int fft_xpass_bin_jobs(int n, const Job* jobs, int njobs, int max_nb, int gx, co
   return set_error(PK_E_INVALID, "unsupported n=%d", n);
 }
 
-int fft_adjoint(int n, const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh, hipStream_t s) {
+int fft_adjoint_grid(int n, int nb) {
   switch (n) {
-#define PK_CASE(V) case V: return FFTLaunch<V>::adjoint(j, tw, coef, bspec, gmesh, s);
+#define PK_CASE(V) case V: return FFTLaunch<V>::adjoint_grid(nb <= HB_LDS);
+    PK_FOR_EACH_N(PK_CASE)
+#undef PK_CASE
+  }
+  return 1;
+}
+
+int fft_adjoint(int n, const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh,
+                double* gsum_part, hipStream_t s) {
+  switch (n) {
+#define PK_CASE(V) case V: return FFTLaunch<V>::adjoint(j, tw, coef, bspec, gmesh, gsum_part, s);
     PK_FOR_EACH_N(PK_CASE)
 #undef PK_CASE
   }

@@ -128,9 +128,18 @@ int fft_ypass_mass(int n, const Job& j, const float2* tw, hipStream_t s);
 int fft_xpass_bin(int n, const Job& j, const float2* tw, int grid, hipStream_t s);
 int bin_finalize(const Job& j, int G, hipStream_t s);
 // backward of the binning: per-bin coefficients coef[nb][3] (float) and j's forward
-// spectrum (after the y pass) -> dLoss/d delta on the mesh gmesh [n][n][n]; bspec is a
-// half-spectrum scratch buffer
-int fft_adjoint(int n, const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh, hipStream_t s);
+// spectrum (after the y pass) -> dLoss/d delta on the mesh gmesh, in bricks (brick_index);
+// bspec is a half-spectrum scratch buffer; gsum_part: fft_adjoint_grid(n, nb) partial sums of
+// g delta over the mesh, g = dLoss/d delta
+int fft_adjoint_grid(int n, int nb);
+int fft_adjoint(int n, const Job& j, const float2* tw, const float* coef, float2* bspec, float* gmesh,
+                double* gsum_part, hipStream_t s);
+// Bricks of 2 x 4 x 4 cells ([x][y][z] inside), one 128-byte line each, C order of the bricks: the
+// 2 x 2 x 2 (3 x 3 x 3) cells of a gather touch 2.3 (4.5) lines on average, 4.1 (9.6) in rows.
+__host__ __device__ inline size_t brick_index(int n, int x, int y, int z) {
+  const size_t b = ((size_t)(x >> 1) * (n >> 2) + (y >> 2)) * (n >> 2) + (z >> 2);
+  return b * 32 + ((x & 1) << 4 | (y & 3) << 2 | (z & 3));
+}
 int ypass_grid(int n);
 int fft_ypass_jobs(int n, const Job* jobs, int njobs, int gy, const float2* tw, hipStream_t s);
 int fft_xpass_bin_jobs(int n, const Job* jobs, int njobs, int max_nb, int gx, const float2* tw, hipStream_t s);
@@ -173,11 +182,11 @@ int scatter_sort_jobs(const Job* jobs, const BatchDims& d, hipStream_t s);
 // coef[b][l] = grad_pk[b][l] norm (2l+1) / counts[b] (0 for empty bins)
 int adjoint_coefficients(const double* grad_pk, const int64_t* counts, int nb, double norm, float* coef,
                          hipStream_t s);
-size_t gather_workspace_bytes(int64_t np);
 // dLoss/d position (grad_pos [np][3], physical units) and dLoss/d weight (nullable) from
-// g = dLoss/d delta on the mesh, through delta = rho n^3 / M - 1 (stats: forward M, n^3 / M)
-int gather_gradients(const ScatterArgs& a, const float* gmesh, const double* stats, float* grad_pos, float* grad_w,
-                     void* ws, size_t ws_bytes, hipStream_t s);
+// g = dLoss/d delta on the mesh (in bricks), through delta = rho n^3 / M - 1 (stats: forward M,
+// n^3 / M); gsum_part: the parts of sum g delta, reduced into *gbar (device)
+int gather_gradients(const ScatterArgs& a, const float* gmesh, const double* stats, const double* gsum_part, int parts,
+                     double* gbar, float* grad_pos, float* grad_w, hipStream_t s);
 
 // ---- fused assignment + z pass (pk_fused.hip) ----------------------------------------------
 // deposit into LDS rows, subtract stats[3], R2C along z, write the spectrum; per-tile
