@@ -50,13 +50,6 @@ template <int N, int TY_> struct FusedCfg {
   static constexpr int WPE = cmax(1, cmin(4, cmax(1, BPC) * (NT / 64) / 4));
 };
 
-// Bucket descriptors of one tile in LDS: first record and exclusive prefix of sizes.
-struct TileBuckets {
-  int base[MAX_TILE_BUCKETS];
-  int pre[MAX_TILE_BUCKETS + 1];
-  int nbk;
-};
-
 // Deposits are rint(W w S) with S = 2^(30 - e), max |w| < 2^e and corner weights W <= 1, so
 // each is below 2^30 and converts through int32; a cell of R records sums below R 2^30 and a
 // tile's cells below 9 R 2^30, inside int64 for any catalogue of < 2^29 particles.  The
@@ -109,39 +102,11 @@ __device__ __forceinline__ void fused_body(const Job& j, int bx, int nbx, const 
   };
   // ... then wave 0 scans the sizes into B (one barrier, which also ends the deposit)
   auto publish = [&](TileBuckets& B, int lo, int hi) {
-    if (tid < 64) {
-      int incl = tid < nbk ? hi - lo : 0;
-#pragma unroll
-      for (int off = 1; off < MAX_TILE_BUCKETS; off <<= 1) {
-        const int v = __shfl_up(incl, off, 64);
-        if (tid >= off) incl += v;
-      }
-      if (tid < nbk) {
-        B.base[tid] = lo;
-        B.pre[tid + 1] = incl;
-      }
-      if (tid == 0) {
-        B.pre[0] = 0;
-        B.nbk = nbk;
-      }
-    }
+    publish_buckets(B, nbk, lo, hi);
     __syncthreads();
   };
-  // record idx of the tile buckets B (clamped to the last one, so the loads of a thread's
-  // records need no branch and are all in flight together; callers test idx < total at the
-  // deposit): a fixed four-step search for the bucket holding idx.  The irregular bucket is
-  // the last one.
-  static_assert(MAX_TILE_BUCKETS <= 16, "four search steps");
-  auto record = [&](const TileBuckets& B, int idx) -> float4 {
-    const int i = min(idx, B.pre[B.nbk] - 1);
-    int b = 0;
-#pragma unroll
-    for (int step = 8; step >= 1; step >>= 1) {
-      const int p = B.pre[b + step];   // b + step <= 15: inside pre[] even beyond nbk
-      b = (b + step < B.nbk && p <= i) ? b + step : b;
-    }
-    return load_record_stream(sorted, (size_t)B.base[b] + (i - B.pre[b]), has_w);
-  };
+  // the irregular bucket is the last one
+  auto record = [&](const TileBuckets& B, int idx) -> float4 { return bucket_record(B, sorted, idx, has_w); };
   auto regular = [&](const TileBuckets& B, int idx) -> bool { return !irregular || idx < B.pre[B.nbk - 1]; };
   // Software pipeline over this block's tiles: the next tile's bucket bounds load during the
   // current deposit, and its first U * NT records are loaded into registers before the

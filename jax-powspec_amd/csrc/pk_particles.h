@@ -385,43 +385,16 @@ __device__ __forceinline__ int row_plane(const ScatterArgs& a, float px, float p
   return home_cell(px, n, stencil);
 }
 
-// Buckets whose particles can deposit into tile (xt, yt): filled into key[] (<= 16).
-__host__ __device__ __forceinline__ int row_tile_buckets(const TileGeom& g, int n, bool tsc, int xt, int yt, int* keys) {
-  int xs[3], nxs = 0;
-  xs[nxs++] = xt;
-  if (n > 1) xs[nxs++] = (xt + n - 1) % n;                 // lower x neighbour (all of it)
-  if (tsc && n > 2) xs[nxs++] = (xt + 1) % n;              // upper x neighbour (TSC)
-  // y: (tile, class) pairs
-  int yc[8], ycl[8], ny = 0;
-  for (int c = 0; c < g.ncls; ++c) { yc[ny] = yt; ycl[ny] = c; ++ny; }
-  if (g.nyt >= 2) {
-    const int lo = (yt + g.nyt - 1) % g.nyt, hi = (yt + 1) % g.nyt;
-    if (tsc) {
-      if (g.nyt >= 3) {
-        yc[ny] = lo; ycl[ny] = 2; ++ny;   // lower tile, last row
-        yc[ny] = hi; ycl[ny] = 1; ++ny;   // upper tile, first row
-      } else {
-        yc[ny] = lo; ycl[ny] = 1; ++ny;   // the other tile's first and last rows
-        yc[ny] = lo; ycl[ny] = 2; ++ny;
-      }
-    } else {
-      yc[ny] = lo; ycl[ny] = 1; ++ny;
-    }
-  }
-  int nk = 0;
-  for (int i = 0; i < nxs; ++i)
-    for (int j = 0; j < ny; ++j) keys[nk++] = (xs[i] * g.nyt + yc[j]) * g.ncls + ycl[j];
-  return nk;
-}
-
-// Number of buckets row_tile_buckets lists (the same for every tile), plus the irregular one.
+// Number of buckets whose particles can deposit into a tile (the same for every tile), plus the
+// irregular one: the tile's own y classes and the boundary-row classes of its y neighbours, in
+// its x plane, the lower one and, for TSC, the upper one.
 __host__ __device__ __forceinline__ int tile_bucket_count(const TileGeom& g, int n, bool tsc, bool irregular) {
   const int nxs = 1 + (n > 1 ? 1 : 0) + (tsc && n > 2 ? 1 : 0);
   const int ny = g.ncls + (g.nyt >= 2 ? (tsc ? 2 : 1) : 0);
   return nxs * ny + (irregular ? 1 : 0);
 }
 
-// Key q of tile (xt, yt) in row_tile_buckets' order; q = nxs * ny is the irregular bucket.
+// Key q of tile (xt, yt); q = nxs * ny is the irregular bucket.
 // Each lane computes its own key, so no lane waits for another before loading key starts.
 __host__ __device__ __forceinline__ int tile_bucket_key(const TileGeom& g, int n, bool tsc, int xt, int yt, int q) {
   const int nxs = 1 + (n > 1 ? 1 : 0) + (tsc && n > 2 ? 1 : 0);
@@ -447,30 +420,47 @@ __host__ __device__ __forceinline__ int tile_bucket_key(const TileGeom& g, int n
   return (x * g.nyt + yc) * g.ncls + ycl;
 }
 
-// Block-cooperative setup of the buckets of tile (xt, yt) (plus the irregular bucket when
-// `irregular`): keys, first record and exclusive prefix of sizes in LDS.  Ends with a barrier.
-__device__ __forceinline__ void gather_buckets(const TileGeom& g, int n, bool tsc, bool irregular, int xt, int yt,
-                                               const int* __restrict__ key_start, int* s_key, int* s_base,
-                                               int* s_pre, int* s_nbk) {
+// Bucket descriptors of one tile in LDS: first record and exclusive prefix of sizes.
+struct TileBuckets {
+  int base[MAX_TILE_BUCKETS];
+  int pre[MAX_TILE_BUCKETS + 1];
+  int nbk;
+};
+static_assert(MAX_TILE_BUCKETS <= 16, "four search steps in bucket_record");
+
+// Wave 0 scans the bucket sizes into B: lane q < nbk holds its bucket's bounds [lo, hi).  The
+// caller's barrier follows.
+__device__ __forceinline__ void publish_buckets(TileBuckets& B, int nbk, int lo, int hi) {
   const int tid = threadIdx.x;
+  if (tid >= 64) return;
+  int incl = tid < nbk ? hi - lo : 0;
+#pragma unroll
+  for (int off = 1; off < MAX_TILE_BUCKETS; off <<= 1) {
+    const int v = __shfl_up(incl, off, 64);
+    if (tid >= off) incl += v;
+  }
+  if (tid < nbk) {
+    B.base[tid] = lo;
+    B.pre[tid + 1] = incl;
+  }
   if (tid == 0) {
-    int nk = row_tile_buckets(g, n, tsc, xt, yt, s_key);
-    if (irregular) s_key[nk++] = g.nkeys - 1;
-    *s_nbk = nk;
+    B.pre[0] = 0;
+    B.nbk = nbk;
   }
-  __syncthreads();
-  const int nk = *s_nbk;
-  if (tid < nk) {
-    const int lo = key_start[s_key[tid]];
-    s_base[tid] = lo;
-    s_pre[tid + 1] = key_start[s_key[tid] + 1] - lo;   // size, prefixed below
+}
+
+// Record idx of the tile buckets B (clamped to the last one, so the loads of a thread's
+// records need no branch and are all in flight together; callers test idx < total at the
+// deposit): a fixed four-step search for the bucket holding idx.
+__device__ __forceinline__ float4 bucket_record(const TileBuckets& B, const void* sorted, int idx, bool has_w) {
+  const int i = min(idx, B.pre[B.nbk] - 1);
+  int b = 0;
+#pragma unroll
+  for (int step = 8; step >= 1; step >>= 1) {
+    const int p = B.pre[b + step];   // b + step <= 15: inside pre[] even beyond nbk
+    b = (b + step < B.nbk && p <= i) ? b + step : b;
   }
-  __syncthreads();
-  if (tid == 0) {
-    s_pre[0] = 0;
-    for (int b = 1; b <= nk; ++b) s_pre[b] += s_pre[b - 1];
-  }
-  __syncthreads();
+  return load_record_stream(sorted, (size_t)B.base[b] + (i - B.pre[b]), has_w);
 }
 
 // 64-bit fixed-point deposit value (two's complement) of a weight already multiplied by
@@ -481,44 +471,5 @@ __device__ __forceinline__ unsigned long long to_fixed(float v) {
   return (unsigned long long)(long long)(int)__builtin_rintf(v);
 }
 __device__ __forceinline__ unsigned long long to_fixed(float wt, float scale) { return to_fixed(wt * scale); }
-
-// Deposit every record of the tile's buckets (set up by gather_buckets) whose corners lie
-// on plane xt and rows [y0, y0 + ty): f(ly, iz, weight).  The bucket of a flat index is
-// found with a register copy of the (<= 17) prefix values.
-template <typename F>
-__device__ __forceinline__ void deposit_buckets(const ScatterArgs& a, const TileGeom& g, const void* sorted,
-                                                const int* s_base, const int* s_pre, int nbk, int nt, int xt, int y0,
-                                                F&& f) {
-  int pre[MAX_TILE_BUCKETS + 1];
-#pragma unroll
-  for (int b = 0; b <= MAX_TILE_BUCKETS; ++b) pre[b] = b <= nbk ? s_pre[b] : 0x7fffffff;
-  const int total = pre[nbk < MAX_TILE_BUCKETS ? nbk : MAX_TILE_BUCKETS];
-  const bool has_w = a.w != nullptr;
-  constexpr int U = 4;   // independent records per thread and iteration (loads in flight)
-  for (int idx0 = threadIdx.x; idx0 < total; idx0 += nt * U) {
-    float4 r[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int idx = idx0 + u * nt;
-      if (idx < total) {
-        int b = 0;
-#pragma unroll
-        for (int j = 1; j < MAX_TILE_BUCKETS; ++j) b += (pre[j] <= idx) ? 1 : 0;
-        r[u] = load_record(sorted, (size_t)s_base[b] + (idx - pre[b]), has_w);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (idx0 + u * nt >= total) continue;
-      auto add = [&](int iy, int iz, float wt) {
-        const int ly = iy - y0;
-        if ((unsigned)ly < (unsigned)g.ty) f(ly, iz, wt);
-      };
-      // the tile buckets hold no irregular record (those are added with global atomics)
-      if (a.stencil == PK_STENCIL_CIC_REF) ref_corners_on_x_regular(a, r[u].x, r[u].y, r[u].z, r[u].w, xt, add);
-      else for_each_corner_on_x(a, r[u].x, r[u].y, r[u].z, r[u].w, xt, add);
-    }
-  }
-}
 
 }  // namespace pk
