@@ -1193,21 +1193,27 @@ __global__ void __launch_bounds__(PAIR_NT) k_bispec_pair(float* __restrict__ p, 
 // delta2), Q = rfftn(I1 I2),
 //   sum_x delta_i^2       = n^-3 sum |D|^2,        sum_x I_i^2     = n^-3 sum 1,
 //   sum_x delta1 delta2 delta_i = n^-3 sum Re(D conj P),  sum_x I1 I2 I_i = n^-3 sum Re Q,
-// so no shell needs its own inverse transform.  Shells s0 .. s0 + ns - 1 (ns <= BKK_CHUNK)
-// per launch, register accumulators, fixed-order block sums into the partial slots.
+// so no shell needs its own inverse transform.
+// Block (x, y) takes 8 shells (chunk y) and rows [kz][kx] of the spectrum, one wave each: a row
+// outside the chunk's shells is left without a read, and of the others only the runs of ky
+// inside them are read (the shells reach a small part of the planes, let alone of the mesh).
+// Register accumulators, fixed-order sums into the partial slots.  20 shells at 256^3: 161 us
+// over all modes of the planes, one launch per 8 shells -> 35 us.
 constexpr int BKK_NT = 256;
 constexpr int BKK_CHUNK = 8;
+constexpr int BKK_WAVES = BKK_NT / 64;
 __global__ void __launch_bounds__(BKK_NT)
 k_bispec_kspace(const float2* __restrict__ dspec, const float2* __restrict__ pspec, const float2* __restrict__ qspec,
-                const float* __restrict__ wt, ShellChunk sh, int s0, int ns, int n, int kz_lim, BispecArgs a) {
-  static_assert(BKK_CHUNK == 8, "ShellChunk holds 8 shells");
-  __shared__ double red[BKK_NT / 64 + 1];
+                const float* __restrict__ wt, ShellTable sh, int first, int count, int n, int kz_lim, BispecArgs a) {
+  __shared__ double part[BKK_WAVES][BKK_CHUNK * 4];
+  const int c0 = blockIdx.y * BKK_CHUNK, ns = min(BKK_CHUNK, count - c0);
+  const int s0 = first + c0;
   int slo[BKK_CHUNK], shi[BKK_CHUNK];
   int mlo = 0x7fffffff, mhi = 0;
 #pragma unroll
   for (int j = 0; j < BKK_CHUNK; ++j) {
-    slo[j] = j < ns ? sh.lo[j] : 1;
-    shi[j] = j < ns ? sh.hi[j] : 0;
+    slo[j] = j < ns ? sh.lo[c0 + j] : 1;
+    shi[j] = j < ns ? sh.hi[c0 + j] : 0;
     if (j < ns) {
       mlo = min(mlo, slo[j]);
       mhi = max(mhi, shi[j]);
@@ -1218,56 +1224,77 @@ k_bispec_kspace(const float2* __restrict__ dspec, const float2* __restrict__ psp
   for (int j = 0; j < BKK_CHUNK; ++j)
 #pragma unroll
     for (int t = 0; t < 4; ++t) acc[j][t] = 0.0;
-  const int h = n / 2;
-  const int64_t nn = (int64_t)n * n;
-  const int64_t total = (int64_t)(kz_lim + 1) * nn;
-  for (int64_t i = (int64_t)blockIdx.x * BKK_NT + threadIdx.x; i < total; i += (int64_t)gridDim.x * BKK_NT) {
-    const int kz = (int)(i / nn);
-    const int r = (int)(i - (int64_t)kz * nn);
-    const int kx = r / n, ky = r - kx * n;
-    const int sx = kx <= h ? kx : kx - n, sy = ky <= h ? ky : ky - n;
-    const int m = sx * sx + sy * sy + kz * kz;
-    if (m < mlo || m >= mhi) continue;
-    const float2 d = dspec[i];
-    const float2 p = pspec[i];
-    const float w = wt[kx] * wt[ky] * wt[kz];
+  const int h = n / 2, lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(blockIdx.x * BKK_WAVES + (threadIdx.x >> 6));
+  const int rows = (kz_lim + 1) * n;
+  for (int row = wave; row < rows; row += gridDim.x * BKK_WAVES) {
+    const int kz = row / n, kx = row - kz * n;
+    const int sx = kx <= h ? kx : kx - n;
+    const int r2 = sx * sx + kz * kz;
+    if (r2 >= mhi) continue;
+    const float wxz = wt[kx] * wt[kz];
     const double wh = (kz == 0 || kz == h) ? 1.0 : 2.0;
-    const double dx = (double)(d.x * w), dy = (double)(d.y * w);
-    const double d2 = wh * (dx * dx + dy * dy);
-    const double tr = wh * (dx * (double)p.x + dy * (double)p.y);
-    const double qq = qspec ? wh * (double)qspec[i].x : 0.0;
+    for (int k0 = 0; k0 < n; k0 += 64) {
+      // |sy| over the run [k0, k1]: smallest and largest
+      const int k1 = min(k0 + 63, n - 1);
+      const int a0 = k0 <= h ? k0 : n - k0, a1 = k1 <= h ? k1 : n - k1;
+      const int amin = k0 == 0 ? 0 : min(a0, a1), amax = k0 <= h && k1 >= h ? h : max(a0, a1);
+      if (r2 + amin * amin >= mhi || r2 + amax * amax < mlo) continue;
+      const int ky = k0 + lane;
+      const int sy = ky <= h ? ky : ky - n;
+      const int m = r2 + sy * sy;
+      if (ky >= n || m < mlo || m >= mhi) continue;
+      const size_t i = (size_t)row * n + ky;
+      const float2 d = dspec[i];
+      const float2 p = pspec[i];
+      const float w = wxz * wt[ky];
+      const double dx = (double)(d.x * w), dy = (double)(d.y * w);
+      const double d2 = wh * (dx * dx + dy * dy);
+      const double tr = wh * (dx * (double)p.x + dy * (double)p.y);
+      const double qq = qspec ? wh * (double)qspec[i].x : 0.0;
 #pragma unroll
-    for (int j = 0; j < BKK_CHUNK; ++j)
-      if (m >= slo[j] && m < shi[j]) {
-        acc[j][0] += d2;
-        acc[j][1] += wh;
-        acc[j][2] += tr;
-        acc[j][3] += qq;
-      }
+      for (int j = 0; j < BKK_CHUNK; ++j)
+        if (m >= slo[j] && m < shi[j]) {
+          acc[j][0] += d2;
+          acc[j][1] += wh;
+          acc[j][2] += tr;
+          acc[j][3] += qq;
+        }
+    }
   }
   const double inv = 1.0 / ((double)n * (double)n * (double)n);
 #pragma unroll
   for (int j = 0; j < BKK_CHUNK; ++j)
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
-      const double v = block_sum_f64_waves<BKK_NT>(acc[j][t], red);
-      __syncthreads();
-      if (j < ns && threadIdx.x == 0)
-        a.part[((size_t)(s0 + j) * BK_SLOTS + t) * BK_PART_STRIDE + blockIdx.x] = v * inv;
+      double v = acc[j][t];
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+      if (lane == 0) part[threadIdx.x >> 6][j * 4 + t] = v;
     }
+  __syncthreads();
+  if (threadIdx.x < BKK_CHUNK * 4 && (int)threadIdx.x / 4 < ns) {
+    double v = 0.0;
+    for (int w = 0; w < BKK_WAVES; ++w) v += part[w][threadIdx.x];
+    a.part[((size_t)(s0 + threadIdx.x / 4) * BK_SLOTS + threadIdx.x % 4) * BK_PART_STRIDE + blockIdx.x] = v * inv;
+  }
 }
 
 constexpr int BKF_NT = 256;
 __global__ void __launch_bounds__(BKF_NT) k_bispec_finalize(BispecArgs a, int n, int g_pair, int g_red) {
   __shared__ double red[BKF_NT / 64 + 1];
   const int sh = blockIdx.x;   // one block per shell (uniform exit)
-  double v[BK_SLOTS];
+  double v[BK_SLOTS] = {0.0, 0.0, 0.0, 0.0};
+  // fixed order: strided per thread, then the block's fixed-order sum
+  const double* pp = a.part + (size_t)sh * BK_SLOTS * BK_PART_STRIDE;
+  const int cnt = sh < 2 ? g_pair : g_red;
+  for (int i = threadIdx.x; i < cnt; i += BKF_NT) {
+#pragma unroll
+    for (int t = 0; t < BK_SLOTS; ++t)
+      if (sh >= 2 || t < 2) v[t] += pp[(size_t)t * BK_PART_STRIDE + i];
+  }
   for (int t = 0; t < BK_SLOTS; ++t) {
-    const int cnt = (sh < 2) ? (t < 2 ? g_pair : 0) : g_red;
-    const double* pp = a.part + ((size_t)sh * BK_SLOTS + t) * BK_PART_STRIDE;
-    double s = 0.0;   // fixed order: strided per thread, then the block's fixed-order sum
-    for (int i = threadIdx.x; i < cnt; i += BKF_NT) s += pp[i];
-    v[t] = block_sum_f64_waves<BKF_NT>(s, red);
+    v[t] = block_sum_f64_waves<BKF_NT>(v[t], red);
     __syncthreads();
   }
   if (threadIdx.x != 0) return;
@@ -1795,7 +1822,7 @@ template <int N> struct FFTLaunch {
   static int kspace_grid() {
     int dev = 0;
     (void)hipGetDevice(&dev);
-    return cmin(BK_PART_STRIDE, num_cus(dev) * 8);
+    return cmin(BK_PART_STRIDE, num_cus(dev) * 2);
   }
   static int pair_grid() {
     static int g = 0;
@@ -1873,15 +1900,16 @@ template <int N> struct FFTLaunch {
       if (!e && !a.i_sums) e = r2c_into(meshes[2], qspec, tw, s, kl);
       if (e) return e;
       gr = kspace_grid();
-      for (int s0 = 2; s0 < a.nshell; s0 += BKK_CHUNK) {
-        const int ns = a.nshell - s0 < BKK_CHUNK ? a.nshell - s0 : BKK_CHUNK;
-        ShellChunk ch{};
-        for (int j = 0; j < ns; ++j) {
-          ch.lo[j] = lo[s0 + j];
-          ch.hi[j] = hi[s0 + j];
+      for (int first = 2; first < a.nshell; first += SHELL_TABLE) {
+        const int count = cmin(SHELL_TABLE, a.nshell - first);
+        ShellTable st{};
+        for (int i = 0; i < count; ++i) {
+          st.lo[i] = lo[first + i];
+          st.hi[i] = hi[first + i];
         }
-        hipLaunchKernelGGL(k_bispec_kspace, dim3(gr), dim3(BKK_NT), 0, s, (const float2*)spec, (const float2*)scratch,
-                           a.i_sums ? nullptr : (const float2*)qspec, wt, ch, s0, ns, N, kl, a);
+        hipLaunchKernelGGL(k_bispec_kspace, dim3(gr, (count + BKK_CHUNK - 1) / BKK_CHUNK), dim3(BKK_NT), 0, s,
+                           (const float2*)spec, (const float2*)scratch, a.i_sums ? nullptr : (const float2*)qspec, wt,
+                           st, first, count, N, kl, a);
       }
     }
     hipLaunchKernelGGL(k_bispec_finalize, dim3(a.nshell), dim3(BKF_NT), 0, s, a, N, gp, gr);

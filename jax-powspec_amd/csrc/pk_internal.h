@@ -247,10 +247,11 @@ struct BispecArgs {
   float* bk;             // [nshell - 2]
   float* qk;             // [nshell - 2]
 };
-// thresholds of up to 8 shells, passed by value to the Fourier-space shell sums
-struct ShellChunk {
-  int lo[8];
-  int hi[8];
+// thresholds of the shells, passed by value to the Fourier-space shell sums
+constexpr int SHELL_TABLE = 128;   // shells per launch
+struct ShellTable {
+  int lo[SHELL_TABLE];
+  int hi[SHELL_TABLE];
 };
 // mesh -> delta_k (r2c into spec) -> the first two shells' fields (masked inverses through
 // scratch) and their products -> spectra of the products (scratch, qspec) -> later shells'
