@@ -154,6 +154,15 @@ template <int M> __device__ __forceinline__ float2 tw_at(TwHalf<M> t, int q) {
   return b ? make_float2(-v.x, -v.y) : v;
 }
 
+// The thread's index, made opaque to the compiler.  Taken once per tile of a persistent block:
+// with the plain index every address and twiddle index of the tile loop is computed once and
+// kept, and the registers cost resident waves or spill.
+__device__ __forceinline__ int opaque_tid() {
+  int t = threadIdx.x;
+  asm volatile("" : "+v"(t));
+  return t;
+}
+
 // ------------------------------------------------------------------------------------
 // One Stockham stage over C independent length-N transforms held in LDS.
 // Element (point p, column c) lives at buf[p * PS + c * CS].  The stage reads radix-R
@@ -205,21 +214,21 @@ __device__ __forceinline__ void fft_stage(float2* buf, TW tw, const int tid = th
 
 template <int N, int S, int NS, int C, int PS, int CS, int NT, bool COLFAST, int TWS, int SK>
 struct FFTStages {
-  template <class TW> static __device__ __forceinline__ void run(float2* buf, TW tw) {
+  template <class TW> static __device__ __forceinline__ void run(float2* buf, TW tw, int tid = threadIdx.x) {
     constexpr int R = radix_at(N, S);
     if constexpr (R > 1) {
-      fft_stage<N, R, NS, C, PS, CS, NT, COLFAST, TWS, SK>(buf, tw);
-      FFTStages<N, S + 1, NS * R, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw);
+      fft_stage<N, R, NS, C, PS, CS, NT, COLFAST, TWS, SK>(buf, tw, tid);
+      FFTStages<N, S + 1, NS * R, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw, tid);
     }
   }
 };
 
 // forward length-N transforms of C columns in LDS (see fft_stage for the layout)
 template <int N, int C, int PS, int CS, int NT, bool COLFAST, int TWS, int SK = 0, class TW>
-__device__ __forceinline__ void lds_fft(float2* buf, TW tw) {
+__device__ __forceinline__ void lds_fft(float2* buf, TW tw, int tid = threadIdx.x) {
   static_assert(fft_size_ok(N), "unsupported FFT length");
   static_assert(SK == 0 || PS == 1, "skewed layouts take unit point stride");
-  FFTStages<N, 0, 1, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw);
+  FFTStages<N, 0, 1, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw, tid);
 }
 
 // ------------------------------------------------------------------------------------
@@ -228,15 +237,8 @@ __device__ __forceinline__ void lds_fft(float2* buf, TW tw) {
 // c = task % C (task = threadIdx.x + t NT): the last stage's outputs of one transform are the
 // first stage's inputs of the next one, if that runs the radices in reverse (REV).  A
 // pointwise step between two transforms then costs no LDS round trip, and neither do the
-// loads and stores of a tile.  tid: the thread's index, made opaque once per tile
-// (opaque_tid): otherwise every address and twiddle index of the tile loop is computed once and
-// kept, and the registers spill.
+// loads and stores of a tile.  tid: opaque_tid(), once per tile.
 // ------------------------------------------------------------------------------------
-__device__ __forceinline__ int opaque_tid() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
 __host__ __device__ constexpr int radix_count(int N) {
   int c = 0;
   while (radix_at(N, c) > 1) ++c;

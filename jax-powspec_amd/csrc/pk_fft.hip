@@ -38,6 +38,12 @@ template <int N> struct FFTCfg {
                      (NTZ / 64) / 4));
 };
 
+// Thread index of the y and z passes' transforms: opaque where the radix-3 plans' kept addresses cost
+// resident waves (384: 211 registers and 2 waves per SIMD in the y pass, 125 and 4 with
+// it; powspec_vec at 384^3 384 -> 358 us).  Elsewhere recomputing them costs more than it
+// gives (512^3: 630 -> 646 us).
+template <int N> __device__ __forceinline__ int pass_tid() { return N % 3 == 0 ? opaque_tid() : (int)threadIdx.x; }
+
 // ------------------------------------------------------------------------------------
 // z pass: real rows -> half spectrum rows, written transposed to [kz][x][y]
 // ------------------------------------------------------------------------------------
@@ -86,7 +92,7 @@ k_zpass(const float* __restrict__ mesh, float2* __restrict__ spec, const float2*
       }
     }
     __syncthreads();
-    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw);
+    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw, pass_tid<N>());
     // split: X[k] = Fe + e^{-2 pi i k / N} Fo, Fe = (Z_k + Z*_{NC-k}) / 2, Fo = -i (Z_k - Z*_{NC-k}) / 2
     // output planes kz <= kz_lim only (callers that read no higher plane pass less than n/2)
     for (int i = tid; i < (min(kz_lim, NC) + 1) * C; i += NT) {
@@ -202,7 +208,7 @@ __device__ __forceinline__ void ypass_body(float2* __restrict__ spec, const floa
     }
     __syncthreads();
     if (item + nbx < NTILES) load(rows.tile(item + nbx));
-    lds_fft<N, C, 1, CS, NT, false, 1, SK>(buf, tw);
+    lds_fft<N, C, 1, CS, NT, false, 1, SK>(buf, tw, pass_tid<N>());
     float2* row = spec + (size_t)tile * C * N;
     const bool streamed = rows.streamed(item);   // block-uniform
     typedef float f2v __attribute__((ext_vector_type(2)));
@@ -1056,7 +1062,7 @@ k_zpass_c2r(const float2* __restrict__ bspec, const float2* __restrict__ twg, fl
       if (kk != k && kk < NC) row[kk] = make_float2(zkk.x, -zkk.y);
     }
     __syncthreads();
-    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw);
+    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw, pass_tid<N>());
     if constexpr (BRICK) {
       // four z of one row per lane, four rows of a brick per 64 bytes
       static_assert(C % 4 == 0 && NC % 2 == 0, "whole brick rows");
@@ -1528,7 +1534,7 @@ k_zpass_c2r_bin(const float2* __restrict__ bspec, const float2* __restrict__ twg
       if (kk != k && kk < NC) row[kk] = make_float2(zkk.x, -zkk.y);
     }
     __syncthreads();
-    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw);
+    lds_fft<NC, C, 1, CS, NT, true, 2>(buf, tw, pass_tid<N>());
     const int sx = x <= H ? x : x - N;
     for (int w = tid; w < BC::RUNS; w += NT) {
       const int c = w / (NC / CH), j0 = (w % (NC / CH)) * CH;
