@@ -231,14 +231,6 @@ __device__ __forceinline__ void lds_fft(float2* buf, TW tw, int tid = threadIdx.
   FFTStages<N, 0, 1, C, PS, CS, NT, COLFAST, TWS, SK>::run(buf, tw, tid);
 }
 
-// ------------------------------------------------------------------------------------
-// Column transforms whose first stage takes its inputs from registers and whose last stage
-// leaves its outputs there.  Both touch rows j + r N / R of column c, for j = task / C and
-// c = task % C (task = threadIdx.x + t NT): the last stage's outputs of one transform are the
-// first stage's inputs of the next one, if that runs the radices in reverse (REV).  A
-// pointwise step between two transforms then costs no LDS round trip, and neither do the
-// loads and stores of a tile.  tid: opaque_tid(), once per tile.
-// ------------------------------------------------------------------------------------
 __host__ __device__ constexpr int radix_count(int N) {
   int c = 0;
   while (radix_at(N, c) > 1) ++c;
@@ -253,6 +245,72 @@ __host__ __device__ constexpr int plan_ns(int N, bool rev, int s) {
   return p;
 }
 
+// Stages S .. E - 1 of the LDS-resident transforms (fft_stage's layout)
+template <int N, int S, int E, int C, int PS, int CS, int NT, bool COLFAST, int TWS, int SK, class TW>
+__device__ __forceinline__ void fft_stages(float2* buf, TW tw) {
+  if constexpr (S < E) {
+    fft_stage<N, radix_at(N, S), plan_ns(N, false, S), C, PS, CS, NT, COLFAST, TWS, SK>(buf, tw);
+    fft_stages<N, S + 1, E, C, PS, CS, NT, COLFAST, TWS, SK>(buf, tw);
+  }
+}
+
+// Last stage of C length-NC transforms of packed real rows (column c at c CS, points
+// consecutive) together with the split into the NC + 1 modes of the real row, in registers:
+// the butterflies j and B - j (B = NC / R of them) hold every pair (k, NC - k) of their outputs, and
+// with fe, t = w^k fo of mode k, X[k] = fe + t and X[NC - k] = conj(fe - t).  Unit 0 takes the
+// butterflies 0 and B / 2, whose pairs lie within themselves.  Saves the stage's LDS write, the
+// split's two reads and a barrier.  tw: e^{-2 pi i q / (2 NC)}.  f(k, c, X) for every mode.
+// B must be even.  A barrier must pass before the LDS is written again.
+template <int NC, int C, int CS, int NT, class F>
+__device__ __forceinline__ void last_stage_split(int tid, const float2* buf, const float2* tw, F&& f) {
+  constexpr int R = radix_at(NC, radix_count(NC) - 1), B = NC / R, UT = B / 2 * C, PER = (UT + NT - 1) / NT;
+  static_assert(B % 2 == 0, "butterflies in pairs");
+  auto emit = [&](int k, int c, float2 zk, float2 zr, bool both) {
+    const float2 fe = make_float2(0.5f * (zk.x + zr.x), 0.5f * (zk.y - zr.y));
+    const float2 fo = make_float2(0.5f * (zk.y + zr.y), -0.5f * (zk.x - zr.x));
+    const float2 t = cmul(tw[k], fo);
+    f(k, c, cadd(fe, t));
+    if (both) f(NC - k, c, make_float2(fe.x - t.x, t.y - fe.y));
+  };
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int task = tid + p * NT;
+    if (UT % NT != 0 && task >= UT) continue;
+    const int u = task / C, c = task % C;
+    const int j1 = u, j2 = u == 0 ? B / 2 : B - u;
+    float2 z1[R], z2[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      z1[r] = buf[c * CS + j1 + r * B];
+      z2[r] = buf[c * CS + j2 + r * B];
+    }
+#pragma unroll
+    for (int r = 1; r < R; ++r) {
+      z1[r] = cmul(z1[r], tw[2 * r * j1]);
+      z2[r] = cmul(z2[r], tw[2 * r * j2]);
+    }
+    DFT<R>::run(z1);
+    DFT<R>::run(z2);
+    if (u != 0) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) emit(j1 + r * B, c, z1[r], z2[R - 1 - r], true);
+    } else {
+#pragma unroll
+      for (int r = 0; 2 * r <= R; ++r) emit(r * B, c, z1[r], z1[r == 0 ? 0 : R - r], 2 * r != R);
+#pragma unroll
+      for (int r = 0; 2 * r <= R - 1; ++r) emit(B / 2 + r * B, c, z2[r], z2[R - 1 - r], 2 * r != R - 1);
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------
+// Column transforms whose first stage takes its inputs from registers and whose last stage
+// leaves its outputs there.  Both touch rows j + r N / R of column c, for j = task / C and
+// c = task % C (task = threadIdx.x + t NT): the last stage's outputs of one transform are the
+// first stage's inputs of the next one, if that runs the radices in reverse (REV).  A
+// pointwise step between two transforms then costs no LDS round trip, and neither do the
+// loads and stores of a tile.  tid: opaque_tid(), once per tile.
+// ------------------------------------------------------------------------------------
 template <int N, int C, int PS, int NT, bool REV> struct ColFFT {
   static constexpr int L = radix_count(N);
   static constexpr int R0 = plan_radix(N, REV, 0);

@@ -40,7 +40,7 @@ template <int N> struct FFTCfg {
 
 // Thread index of the y and z passes' transforms: opaque where the radix-3 plans' kept addresses cost
 // resident waves (384: 211 registers and 2 waves per SIMD in the y pass, 125 and 4 with
-// it; powspec_vec at 384^3 384 -> 358 us).  Elsewhere recomputing them costs more than it
+// it; powspec_vec at 384^3 387 -> 349 us).  Elsewhere recomputing them costs more than it
 // gives (512^3: 630 -> 646 us).
 template <int N> __device__ __forceinline__ int pass_tid() { return N % 3 == 0 ? opaque_tid() : (int)threadIdx.x; }
 

@@ -45,7 +45,12 @@ template <int N, int TY_> struct FusedCfg {
   // waves: the mass and square sums go by wave.
   static constexpr int NT0 = cmin(1024, cmax(cmin(512, (TY * N + 63) / 64 * 64), (TY * NC / 8) / 64 * 64));
   static constexpr int NT = BPC >= 2 ? cmin(NT0, 512) : NT0;
-  static constexpr int PER = (TY * N + NT - 1) / NT;     // cells per thread in the conversion
+  // The last stage and the split in registers (last_stage_split) where their units occupy every
+  // thread: whole estimates 986 -> 963 us at 512^3 (2e7 particles), 2730 -> 2594 at 768^3 (1e7),
+  // 515 -> 505 at 384^3 (3e6, TSC).  At 1024 they would occupy half: 6420 -> 6510 us.
+  static constexpr int L = radix_count(NC);
+  static constexpr int BL = NC / radix_at(NC, L - 1);    // butterflies of the last stage
+  static constexpr bool REG_SPLIT = L >= 2 && BL % 2 == 0 && BL / 2 * TY >= NT;
   // waves per SIMD the LDS allows (capped at 4): the register budget is held to it
   static constexpr int WPE = cmax(1, cmin(4, cmax(1, BPC) * (NT / 64) / 4));
 };
@@ -240,17 +245,23 @@ __device__ __forceinline__ void fused_body(const Job& j, int bx, int nbx, const 
         }
       }
       __syncthreads();
-      FFTStages<NC, 1, R0, C, 1, CS, NT, true, 2, 0>::run(buf, tw);
-    }
-    for (int i = tid; i < (NC + 1) * C; i += NT) {
-      const int c = i % C, k = i / C;
-      const float2 zk = buf[c * CS + (k == NC ? 0 : k)];
-      const float2 zr = buf[c * CS + (k == 0 ? 0 : NC - k)];
-      const float2 zc = make_float2(zr.x, -zr.y);
-      const float2 fe = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
-      const float2 dd = csub(zk, zc);
-      const float2 fo = make_float2(0.5f * dd.y, -0.5f * dd.x);
-      spec[((size_t)k * N + xt) * N + (size_t)y0 + c] = cadd(fe, cmul(tw[k], fo));
+      auto store = [&](int k, int c, float2 X) { spec[((size_t)k * N + xt) * N + (size_t)y0 + c] = X; };
+      if constexpr (Cf::REG_SPLIT) {
+        fft_stages<NC, 1, Cf::L - 1, C, 1, CS, NT, true, 2, 0>(buf, tw);
+        last_stage_split<NC, C, CS, NT>(opaque_tid(), buf, tw, store);
+      } else {
+        FFTStages<NC, 1, R0, C, 1, CS, NT, true, 2, 0>::run(buf, tw);
+        for (int i = tid; i < (NC + 1) * C; i += NT) {
+          const int c = i % C, k = i / C;
+          const float2 zk = buf[c * CS + (k == NC ? 0 : k)];
+          const float2 zr = buf[c * CS + (k == 0 ? 0 : NC - k)];
+          const float2 zc = make_float2(zr.x, -zr.y);
+          const float2 fe = make_float2(0.5f * (zk.x + zc.x), 0.5f * (zk.y + zc.y));
+          const float2 dd = csub(zk, zc);
+          const float2 fo = make_float2(0.5f * dd.y, -0.5f * dd.x);
+          store(k, c, cadd(fe, cmul(tw[k], fo)));
+        }
+      }
     }
     __syncthreads();   // the split has read the rows before the next tile clears them
     t_prev = t;
