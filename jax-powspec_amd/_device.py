@@ -77,6 +77,22 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)
 
 
+def upload(a, device: torch.device) -> torch.Tensor:
+    """A small host array on the device, in the order of the current stream.
+
+    Through pinned memory the call returns at once: a copy from pageable memory holds the host
+    until the stream has run everything before it, which serialises back-to-back calls.  (Under
+    capture the copy stays a pageable one, which the capture refuses: a replay would read a
+    pinned block that has gone to another use.)
+    """
+    src = torch.from_numpy(np.ascontiguousarray(a))
+    if torch.cuda.is_current_stream_capturing():
+        return src.to(device)
+    pinned = torch.empty(src.shape, dtype=src.dtype, pin_memory=True)
+    pinned.copy_(src)
+    return pinned.to(device, non_blocking=True)
+
+
 def as_f32_vector(a, device: torch.device, name: str) -> tuple[torch.Tensor, int]:
     """1-D float32 device view (no copy when already one) and its element stride."""
     if isinstance(a, torch.Tensor):

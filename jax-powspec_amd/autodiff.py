@@ -125,5 +125,5 @@ def estimate_ad(pos, w=None, *, box_size, n_bins, k_edges=None, mas="CIC_REF", w
     if fundamental:
         k3D = (kmean.detach() * kF).to(torch.float32)
     else:
-        k3D = torch.as_tensor((0.5 * (edges[1:] + edges[:-1]) * kF).astype(np.float32), device=device)
+        k3D = _device.upload((0.5 * (edges[1:] + edges[:-1]) * kF).astype(np.float32), device)
     return k3D, pk, nmodes

@@ -204,14 +204,24 @@ class BatchEstimator:
         self.knobs = (int(count_rounds), int(ypass_pct), int(xpass_pct))
         return self
 
-    def result(self, i: int, full: bool = False):
+    def _centres(self, indices):
+        """Bin centres (float32, device) of the jobs whose edges were given, in one copy; None for
+        fundamental bins."""
+        host = {i: (0.5 * (j.edges[1:] + j.edges[:-1]) * (2.0 * np.pi / j.box)).astype(np.float32)
+                for i, j in ((i, self.jobs[i]) for i in indices) if not j.fundamental}
+        if not host:
+            return {}
+        parts = _device.upload(np.concatenate(list(host.values())), self.device).split([a.size for a in host.values()])
+        return dict(zip(host, parts))
+
+    def result(self, i: int, full: bool = False, _k3D=None):
         j = self.jobs[i]
         nb = j.nb
         kF = 2.0 * np.pi / j.box
         if j.fundamental:
             k3D = (self.kmean[i, :nb] * kF).to(torch.float32)
         else:
-            k3D = torch.as_tensor((0.5 * (j.edges[1:] + j.edges[:-1]) * kF).astype(np.float32), device=self.device)
+            k3D = _k3D if _k3D is not None else self._centres([i])[i]
         res = (k3D, self.pk[i, :nb], self.nmodes[i, :nb])
         if full:
             extras = {"sums": self.sums[i, :nb], "counts": self.counts[i, :nb],
@@ -222,7 +232,8 @@ class BatchEstimator:
         return res
 
     def results(self, full: bool = False):
-        return [self.result(i, full) for i in range(len(self.jobs))]
+        k = self._centres(range(len(self.jobs)))
+        return [self.result(i, full, k.get(i)) for i in range(len(self.jobs))]
 
 
 def run_concurrent(batches, *, stream=None):

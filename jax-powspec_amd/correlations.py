@@ -98,7 +98,7 @@ def powspec_vec(delta, box_size, k_edges, *, mas="CIC", shot_noise=0.0, full=Fal
     flags = _lib.FLAG_KMEAN if full else 0
     out, device = _powspec(delta, box_size, e, p=_window_p(mas), shot_noise=shot_noise, flags=flags)
     kF = 2.0 * np.pi / float(box_size)
-    k3D = torch.as_tensor((0.5 * (e[1:] + e[:-1]) * kF).astype(np.float32), device=device)
+    k3D = _device.upload((0.5 * (e[1:] + e[:-1]) * kF).astype(np.float32), device)
     res = (k3D, out.pk, out.nmodes)
     return res + (_extras(out, kF),) if full else res
 
@@ -170,7 +170,7 @@ def xi_vec(delta, box_size, s_edges, *, mas="CIC", full=False):
     n = int(delta.shape[0])
     e = np.asarray(s_edges, np.float64).reshape(-1) * n / float(box_size)
     xi, nm, sums, tab, device = _xi(delta, e, _window_p(mas), 0)
-    r = torch.as_tensor((0.5 * (e[1:] + e[:-1]) * (float(box_size) / n)).astype(np.float32), device=device)
+    r = _device.upload((0.5 * (e[1:] + e[:-1]) * (float(box_size) / n)).astype(np.float32), device)
     res = (r, xi, nm)
     return res + ({"sums": sums, "counts": tab.modes},) if full else res
 
@@ -245,8 +245,8 @@ def bispec(delta, box_size, k1, k2, theta, *, mas="CIC", full=False, reuse_shell
             if len(_BISPEC_I_SUMS) > 256:
                 _BISPEC_I_SUMS.clear()
             _BISPEC_I_SUMS[key] = sums[:, [1, 3]].contiguous()
-    f32 = lambda a: torch.as_tensor(np.asarray(a, np.float32), device=device)
-    res = (f32(k_all), pk, f32(th), bk[:ns - 2], qk[:ns - 2])
+    kt = _device.upload(np.concatenate([k_all, th]).astype(np.float32), device)   # one copy for both
+    res = (kt[:ns], pk, kt[ns:], bk[:ns - 2], qk[:ns - 2])
     return res + ({"sums": sums, "shell_lo": lo, "shell_hi": hi},) if full else res
 
 
@@ -318,7 +318,7 @@ def estimate(x, y, z, w=None, *, box_size, n_bins, k_edges=None, mas="CIC_REF", 
     if fundamental:
         k3D = (out.kmean * kF).to(torch.float32)
     else:
-        k3D = torch.as_tensor((0.5 * (e[1:] + e[:-1]) * kF).astype(np.float32), device=device)
+        k3D = _device.upload((0.5 * (e[1:] + e[:-1]) * kF).astype(np.float32), device)
     res = (k3D, out.pk, out.nmodes)
     return res + (_extras(out, kF),) if full else res
 

@@ -46,7 +46,8 @@ def _pk_table(kf, Pkf, device):
         raise ValueError("kf and Pkf must be 1-D tables of the same length >= 2")
     if not np.all(np.diff(kf) > 0):
         raise ValueError("kf must be strictly increasing")
-    return (torch.as_tensor(kf, device=device), torch.as_tensor(pk, device=device), int(kf.size))
+    both = _device.upload(np.concatenate([kf, pk]), device)   # one copy for both
+    return both[:kf.size], both[kf.size:], int(kf.size)
 
 
 def _field_ws(n, device):
