@@ -858,6 +858,10 @@ int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g,
     // 768 and 1024: 16)
     ty = largest_divisor_le(n, 32);
     while (ty > 2 && ((size_t)ty * n * 8 > FIXED_LDS_MAX || n % ty != 0)) --ty;
+    if (n % ty != 0) {   // no divisor's rows fit (odd sides above 127 without one up to 32): global atomics
+      *direct = true;
+      return PK_OK;
+    }
   }
   g->ty = ty;
   g->nyt = n / ty;
