@@ -45,12 +45,13 @@ template <int N, int TY_> struct FusedCfg {
   // waves: the mass and square sums go by wave.
   static constexpr int NT0 = cmin(1024, cmax(cmin(512, (TY * N + 63) / 64 * 64), (TY * NC / 8) / 64 * 64));
   static constexpr int NT = BPC >= 2 ? cmin(NT0, 512) : NT0;
-  // The last stage and the split in registers (last_stage_split) where their units occupy every
-  // thread: whole estimates 986 -> 963 us at 512^3 (2e7 particles), 2730 -> 2594 at 768^3 (1e7),
-  // 515 -> 505 at 384^3 (3e6, TSC).  At 1024 they would occupy half: 6420 -> 6510 us.
+  // The last stage and the split in registers (last_stage_split) where their units occupy two
+  // thirds of the threads or more: whole estimates 986 -> 963 us at 512^3 (2e7 particles), 515 ->
+  // 505 at 384^3 (3e6, TSC), 2614 -> 2531 at 768^3 (1e7, two thirds).  At 1024 they would occupy
+  // half: 6420 -> 6510 us.
   static constexpr int L = radix_count(NC);
   static constexpr int BL = NC / radix_at(NC, L - 1);    // butterflies of the last stage
-  static constexpr bool REG_SPLIT = L >= 2 && BL % 2 == 0 && BL / 2 * TY >= NT;
+  static constexpr bool REG_SPLIT = L >= 2 && BL % 2 == 0 && BL / 2 * TY * 3 >= NT * 2;
   // waves per SIMD the LDS allows (capped at 4): the register budget is held to it
   static constexpr int WPE = cmax(1, cmin(4, cmax(1, BPC) * (NT / 64) / 4));
 };
