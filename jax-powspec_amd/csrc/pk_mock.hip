@@ -7,7 +7,7 @@
 //   sum   : FP64 per-block sums of rho = exp(bias * field) (or field) -> fixed-order total
 //   count : Poisson counts per cell (one byte each, saturated) -> per-block totals ->
 //           exclusive scan (block offsets)
-//   emit  : the block scans its cells' stored counts and lists its particles' cells in LDS,
+//   emit  : the block scans its cells' stored counts and finds its particles' cells in LDS,
 //           then one thread per particle: draws, offset, shift, wrap, the (x, y, z) record
 // A block owns POP_CELLS consecutive cells in C order (the count visits them in rounds of
 // 2 POP_NT, a thread taking a pair, whose two Poisson draws share one Philox block), so
@@ -28,7 +28,7 @@ constexpr int POP_ROUNDS = 8;
 constexpr int POP_CELLS = 2 * POP_NT * POP_ROUNDS;
 constexpr int TOP_NT = 1024;
 constexpr int TOP_ROWS = 8;   // block totals per thread in flight
-constexpr int MISC_LEN = 4;   // [0] rate scale, [1] total (as int64 bits), [2] sum rho
+constexpr int MISC_LEN = 4;   // [0] rate scale, [1] total (as int64 bits), [2] sum rho, [3] lengths of the lists of dense and of saturated blocks (two ints)
 
 int64_t pop_blocks(int n) {
   const int64_t nc = (int64_t)n * n * n;
@@ -222,6 +222,7 @@ __global__ void __launch_bounds__(TOP_NT) k_pop_scale(PopK a) {
   if (threadIdx.x == 0) {
     a.misc[0] = a.mean_obj / (t / (double)a.ncell);
     a.misc[2] = t;
+    a.misc[3] = 0.0;   // no block is listed yet
   }
 }
 
@@ -232,25 +233,61 @@ __device__ __forceinline__ void pair_counts(const PopK& a, int64_t c, double sca
   poisson_pair(l0, l1, (uint64_t)c, a.k0, a.k1, n0, n1);
 }
 
+// orders a wave's LDS writes before its lanes' later reads of them
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// How a block of cells is emitted (k_pop_emit): by the most particles that EMIT_PER consecutive cells
+// (one thread of the emitting block) hold, at most EMIT_OWN or more, and whether a count is saturated
+enum { EMIT_SPARSE = 0, EMIT_DENSE = 1, EMIT_SATURATED = 2 };
+constexpr int EMIT_PER = POP_CELLS / POP_NT;   // cells per thread
+constexpr int EMIT_OWN = 64;
+
+// The field's sums are spent once the rate scale is known: their place holds [nblk] block routes and
+// [nblk] block numbers, the dense ones from the front and the saturated ones from the back; misc[3]
+// their two lengths.
+__device__ __forceinline__ int* pop_route(const PopK& a) { return reinterpret_cast<int*>(a.rsum); }
+__device__ __forceinline__ int* pop_listed(const PopK& a, bool sat, int i) {
+  return reinterpret_cast<int*>(a.rsum) + a.nblk + (sat ? a.nblk - 1 - i : i);
+}
+__device__ __forceinline__ int* pop_list_length(const PopK& a, bool sat) {
+  return reinterpret_cast<int*>(a.misc + 3) + (sat ? 1 : 0);
+}
+
+// particles of the 16 cells whose stored counts are (lo, hi)
+__device__ __forceinline__ int bytes_sum(uint64_t lo, uint64_t hi) {
+  uint32_t s = __builtin_amdgcn_sad_u8((uint32_t)lo, 0u, 0u);
+  s = __builtin_amdgcn_sad_u8((uint32_t)(lo >> 32), 0u, s);
+  s = __builtin_amdgcn_sad_u8((uint32_t)hi, 0u, s);
+  return (int)__builtin_amdgcn_sad_u8((uint32_t)(hi >> 32), 0u, s);
+}
+// whether a byte of v is 255
+__device__ __forceinline__ bool any_saturated(uint64_t v) {
+  constexpr uint64_t LOW = 0x7f7f7f7f7f7f7f7full, TOP = 0x8080808080808080ull;
+  return (((v & LOW) + 0x0101010101010101ull) & v & TOP) != 0;
+}
+
 // Most cells hold no particle, and u <= 1 - lambda decides that without exp(-lambda): 1 - lambda
 // <= exp(-lambda), and the margin of 2^-50 covers the rounding of both.  The other cells go to a
 // list in LDS, whose draws (the exponential and the inversion loop, or the rejection) then
-// run with full waves.  Counts equal those of a draw per cell.  512^3 cells, 2e7 particles:
-// 829 -> 667 us.
-constexpr int CNT_LIST = 4 * POP_NT;   // a round adds at most 2 POP_NT
+// run with full waves.  Counts equal those of a draw per cell.  512^3 cells, 2e7 particles, bias 1 of
+// a unit Gaussian field: a draw per cell 692 us, one list per block 582, a list per wave (no round
+// waits for another wave) 547; 64^3 cells with half a particle each: 11.8, 15.4 and 13.3 us.
+constexpr int CNT_LIST = 256;   // entries per wave; a round adds at most 128
 __global__ void __launch_bounds__(POP_NT) k_pop_count(PopK a) {
-  __shared__ long long red[POP_NT / 64];
-  __shared__ double list_l[CNT_LIST], list_u[CNT_LIST];
-  __shared__ uint16_t list_c[CNT_LIST];
+  constexpr int NW = POP_NT / 64;
+  __shared__ long long red[NW];
+  __shared__ double list_l[NW][CNT_LIST], list_u[NW][CNT_LIST];
+  __shared__ uint16_t list_c[NW][CNT_LIST];
   __shared__ __align__(16) uint8_t cnt[POP_CELLS];   // saturated: 255 means "recount"
-  __shared__ int nlist;
-  const int tid = threadIdx.x, lane = tid & 63;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const double scale = a.misc[0];
   const int64_t c0 = (int64_t)blockIdx.x * POP_CELLS;
-  for (int i = tid; i < POP_CELLS / 16; i += POP_NT) reinterpret_cast<uint4*>(cnt)[i] = make_uint4(0u, 0u, 0u, 0u);
-  if (tid == 0) nlist = 0;
-  __syncthreads();
-  long long s = 0;   // counts (at most 2^42 in a block), and saturated cells from bit 48
+  static_assert(EMIT_PER == 16, "one 16-byte access of counts per thread");
+  reinterpret_cast<uint4*>(cnt)[tid] = make_uint4(0u, 0u, 0u, 0u);
   float f0, f1;
   auto load = [&](int k) {
     const int64_t c = pop_pair(k);
@@ -258,6 +295,9 @@ __global__ void __launch_bounds__(POP_NT) k_pop_count(PopK a) {
     f1 = c + 1 < a.ncell ? a.field[c + 1] : 0.0f;
   };
   load(0);
+  __syncthreads();
+  long long s = 0;   // counts: at most 2^42 in a block
+  int have = 0;      // the wave's listed cells
 #pragma unroll 1
   for (int k = 0; k < POP_ROUNDS; ++k) {
     const int64_t c = pop_pair(k);
@@ -270,43 +310,44 @@ __global__ void __launch_bounds__(POP_NT) k_pop_count(PopK a) {
     for (int e = 0; e < 2; ++e) {
       const bool draw = lam[e] > 0.0 && !(u[e] + 0x1p-50 <= 1.0 - lam[e]);
       const uint64_t m = __ballot(draw);
-      if (m == 0) continue;   // wave-uniform
-      int base = 0;
-      if (lane == 0) base = atomicAdd(&nlist, __popcll(m));
-      base = __shfl(base, 0, 64);
       if (draw) {
-        const int at = base + __popcll(m & ((1ull << lane) - 1));
-        list_l[at] = lam[e];
-        list_u[at] = u[e];
-        list_c[at] = (uint16_t)(c + e - c0);
+        const int at = have + __popcll(m & ((1ull << lane) - 1));
+        list_l[wv][at] = lam[e];
+        list_u[wv][at] = u[e];
+        list_c[wv][at] = (uint16_t)(c + e - c0);
       }
+      have += __popcll(m);
     }
-    __syncthreads();
-    const int have = nlist;
-    if (have > CNT_LIST - 2 * POP_NT || k + 1 == POP_ROUNDS) {   // block-uniform
-      for (int i = tid; i < have; i += POP_NT) {
-        const int at = list_c[i];
-        const int n = poisson_draw(list_l[i], list_u[i], (uint64_t)(c0 + at), a.k0, a.k1);
+    if (have > CNT_LIST - 128 || k + 1 == POP_ROUNDS) {   // wave-uniform
+      wave_lds_fence();
+      for (int i = lane; i < have; i += 64) {
+        const int at = list_c[wv][i];
+        const int n = poisson_draw(list_l[wv][i], list_u[wv][i], (uint64_t)(c0 + at), a.k0, a.k1);
         cnt[at] = (uint8_t)min(n, 255);
-        s += (long long)n + (n >= 255 ? 1ll << 48 : 0ll);
+        s += n;
       }
-      __syncthreads();
-      if (tid == 0) nlist = 0;
+      wave_lds_fence();
+      have = 0;
     }
-    __syncthreads();   // every thread has read the list's length before the next round adds to it
   }
+  __syncthreads();
+  const ulonglong2 mine = reinterpret_cast<const ulonglong2*>(cnt)[tid];
+  if (bytes_sum(mine.x, mine.y) > EMIT_OWN) s += 1ll << 43;              // at most 2^51 in a block
+  if (any_saturated(mine.x) || any_saturated(mine.y)) s += 1ll << 52;
   // whole pairs, the mesh's last one too (its second cell counts 0)
   const int64_t pairs = min((int64_t)POP_CELLS, a.ncell - c0 + 1) / 2;
   if (pairs == POP_CELLS / 2) {
-    for (int i = tid; i < POP_CELLS / 16; i += POP_NT)
-      reinterpret_cast<uint4*>(a.cnt + c0 / 2)[i] = reinterpret_cast<const uint4*>(cnt)[i];
+    reinterpret_cast<ulonglong2*>(a.cnt + c0 / 2)[tid] = mine;
   } else {
     for (int i = tid; i < pairs; i += POP_NT) a.cnt[c0 / 2 + i] = reinterpret_cast<const uint16_t*>(cnt)[i];
   }
   const long long t = block_sum_i64(s, red);
   if (tid == 0) {
-    a.boff[blockIdx.x] = t & ((1ll << 48) - 1);
-    a.rsum[blockIdx.x] = t >> 48 ? 1.0 : 0.0;   // the field's sums are spent: whether a count is saturated
+    a.boff[blockIdx.x] = t & ((1ll << 43) - 1);
+    const int route = t >> 52 ? EMIT_SATURATED : t >> 43 ? EMIT_DENSE : EMIT_SPARSE;
+    pop_route(a)[blockIdx.x] = route;
+    const bool sat = route == EMIT_SATURATED;
+    if (route != EMIT_SPARSE) *pop_listed(a, sat, atomicAdd(pop_list_length(a, sat), 1)) = blockIdx.x;
   }
 }
 
@@ -331,10 +372,12 @@ __global__ void __launch_bounds__(TOP_NT) k_pop_scan(PopK a) {
 #pragma unroll
     for (int r = 0; r < TOP_ROWS; ++r) {
       incl[r] = v[r];
+      if (b0 + r * TOP_NT < a.nblk) {   // block-uniform
 #pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const long long t = __shfl_up(incl[r], off, 64);
-        if (lane >= off) incl[r] += t;
+        for (int off = 1; off < 64; off <<= 1) {
+          const long long t = __shfl_up(incl[r], off, 64);
+          if (lane >= off) incl[r] += t;
+        }
       }
       if (lane == 63) wt[r * NW + w] = incl[r];
     }
@@ -379,107 +422,162 @@ __device__ __forceinline__ float wrap_box(double r, double box) {
   return f >= (float)box ? 0.0f : f;
 }
 
-// The block's particles: a thread scans 16 consecutive cells' counts (one 16-byte load), the block
-// scans the threads' sums, every thread lists its particles' cells in LDS (EMIT_WIN slots at a
-// time), and the lanes then take consecutive particles: cell centre + triangular offset
-// (+ redshift-space shift), wrapped into [0, L).  Marking the cells in the output records in one
-// kernel and turning them into positions in another took 406 + 163 us for 2e7 particles at
-// 512^3; now 286 us and 72 us for the blocks with saturated counts.
-// SAT: the blocks that hold a saturated count, whose recount takes the Poisson draws' registers (138
-// against 50: 505 us for one kernel of both); the others in a launch without it.
-constexpr int EMIT_WIN = 4096;
-constexpr int EMIT_SAT_BLOCKS = 8192;
-constexpr int EMIT_PER = POP_CELLS / POP_NT;   // cells per thread
-template <bool SAT>
-__device__ __forceinline__ void pop_emit_body(const PopK& a, int blk) {
-  static_assert(EMIT_PER == 16, "one 16-byte load of counts per thread");
-  __shared__ long long sh[POP_NT / 64];
-  __shared__ uint16_t list[EMIT_WIN];   // cell of each slot, from the block's first
-  const int64_t c0 = (int64_t)blk * POP_CELLS;
-  const int64_t mine = c0 + (int64_t)threadIdx.x * EMIT_PER;
-  const long long base = a.boff[blk];
-  // counts of the thread's cells: stored bytes; 255 means recount (any may be saturated)
-  uint64_t lo = 0, hi = 0;
-  if (mine + EMIT_PER <= a.ncell) {
-    const ulonglong2 v = reinterpret_cast<const ulonglong2*>(a.cnt)[mine / EMIT_PER];
-    lo = v.x;
-    hi = v.y;
-  } else {
-    for (int i = 0; i < EMIT_PER; ++i)
-      if (mine + i < a.ncell) {
-        const uint64_t pair = a.cnt[(mine + i) >> 1];   // the cell's byte of its pair
-        (i < 8 ? lo : hi) |= ((i & 1 ? pair >> 8 : pair) & 255u) << (8 * (i & 7));
-      }
-  }
-  // f(i, count) for the thread's cells that hold particles, in order
-  auto each_count = [&](auto&& f) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      uint64_t left = h ? hi : lo;
-#pragma unroll 1
-      while (left) {
-        const int k = (__ffsll((unsigned long long)left) - 1) >> 3;
-        const uint64_t byte = 255ull << (8 * k);
-        long long n = (long long)((left & byte) >> (8 * k));
-        left &= ~byte;
-        if constexpr (SAT) {
-          if (n == 255) {
-            int n0, n1;
-            const int64_t c = mine + 8 * h + k;
-            pair_counts(a, c & ~(int64_t)1, a.misc[0], n0, n1);
-            n = c & 1 ? n1 : n0;
-          }
-        }
-        f(8 * h + k, n);
-      }
-    }
-  };
-  long long own = 0;
-  if constexpr (SAT) {
-    each_count([&](int, long long n) { own += n; });
-  } else {   // sums of four bytes each
-    own = __builtin_amdgcn_sad_u8((uint32_t)lo, 0u, 0u);
-    own = __builtin_amdgcn_sad_u8((uint32_t)(lo >> 32), 0u, (uint32_t)own);
-    own = __builtin_amdgcn_sad_u8((uint32_t)hi, 0u, (uint32_t)own);
-    own = __builtin_amdgcn_sad_u8((uint32_t)(hi >> 32), 0u, (uint32_t)own);
-  }
-  long long total;
-  const long long first = block_scan_i64<POP_NT>(own, sh, total);   // this thread's first slot
+// One particle: output slot p, cell c
+__device__ __forceinline__ void emit_particle(const PopK& a, long long p, uint32_t c) {
   const uint32_t n = (uint32_t)a.n;
-  for (long long w0 = 0; w0 < total; w0 += EMIT_WIN) {   // block-uniform
-    const long long w1 = min(w0 + (long long)EMIT_WIN, total);
+  const uint32_t iz = c % n, cy = c / n;
+  const uint32_t iy = cy % n, ix = cy / n;
+  const Philox4 w = rng_block((uint64_t)p, 0, TAG_DISP, a.k0, a.k1);
+  const double shift = (a.psi != nullptr && a.growth != 0.0) ? a.growth * (double)a.psi[c] : 0.0;
+  typedef float f3 __attribute__((ext_vector_type(3), aligned(4)));
+  const f3 f = {wrap_box(((double)ix + 0.5 + tri_offset(w.x)) * a.H, a.box),
+                wrap_box(((double)iy + 0.5 + tri_offset(w.y)) * a.H, a.box),
+                wrap_box(((double)iz + 0.5 + tri_offset(w.z)) * a.H + shift, a.box)};
+  *reinterpret_cast<f3*>(a.pos + 3 * p) = f;
+}
+
+// stored counts of the thread's EMIT_PER consecutive cells of block blk
+__device__ __forceinline__ ulonglong2 load_counts(const PopK& a, int blk) {
+  const int64_t mine = (int64_t)blk * POP_CELLS + (int64_t)threadIdx.x * EMIT_PER;
+  if (mine + EMIT_PER <= a.ncell) return reinterpret_cast<const ulonglong2*>(a.cnt)[mine / EMIT_PER];
+  ulonglong2 v = {0, 0};
+  for (int i = 0; i < EMIT_PER; ++i)
+    if (mine + i < a.ncell) {
+      const uint64_t pair = a.cnt[(mine + i) >> 1];   // the cell's byte of its pair
+      (i < 8 ? v.x : v.y) |= ((i & 1 ? pair >> 8 : pair) & 255u) << (8 * (i & 7));
+    }
+  return v;
+}
+
+// Emission, by what the block's cells hold.  Bound by the draws and FP64 arithmetic of the particles
+// where the finding of their cells keeps up: a thread that lists its cells' particles one by one holds
+// up its block once they are many (64^3 cells of 40 particles: 1112 us, against 225 to mark the slots
+// from the waves and 84 to emit), so blocks with more than EMIT_OWN in the cells of one thread go by
+// bisection (119 us there).  Whole calls, us, marking / listing alone / both ways as here:
+// 64^3 cells of 40: 395 / 1228 / 208; of 300: 2346 / 35700 / 1234; 128^3, 1 per cell, bias 2: 146 /
+// 215 / 129; 256^3 of 2: 563 / 470 / 457 (EMIT_OWN 32: 514); 256^3 of 0.15: 175 / 139 / 126.  At 512^3
+// with 2e7 particles marking and emitting take 407 + 158 us, this 253 + 4.
+// Sparse blocks: a thread scans its 16 cells' counts (one 16-byte load), the block scans the threads'
+// sums, every thread lists its particles' cells in LDS (EMIT_WIN slots at a time), and the lanes then
+// take consecutive particles.
+constexpr int EMIT_WIN = 4096;
+__device__ __forceinline__ void emit_sparse(const PopK& a, int blk, uint16_t* list) {
+  __shared__ long long sh[POP_NT / 64];
+  const int64_t c0 = (int64_t)blk * POP_CELLS;
+  const long long base = a.boff[blk];
+  const ulonglong2 v = load_counts(a, blk);
+  const int own = bytes_sum(v.x, v.y);
+  long long sum;
+  const int first = (int)block_scan_i64<POP_NT>(own, sh, sum);   // this thread's first slot
+  const int total = (int)sum;
+  for (int w0 = 0; w0 < total; w0 += EMIT_WIN) {   // block-uniform
+    const int w1 = min(w0 + EMIT_WIN, total);
     if (own > 0 && first < w1 && first + own > w0) {
-      long long s = first;
-      each_count([&](int i, long long n) {
-        for (long long q = max(s, w0); q < min(s + n, w1); ++q)
-          list[q - w0] = (uint16_t)(threadIdx.x * EMIT_PER + i);
-        s += n;
-      });
+      int s = first;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        uint64_t left = h ? v.y : v.x;
+#pragma unroll 1
+        while (left) {
+          const int k = (__ffsll((unsigned long long)left) - 1) >> 3;
+          const int end = s + (int)((left >> (8 * k)) & 255u);
+          left &= ~(255ull << (8 * k));
+          for (int q = max(s, w0); q < min(end, w1); ++q) list[q - w0] = (uint16_t)(threadIdx.x * EMIT_PER + 8 * h + k);
+          s = end;
+        }
+      }
     }
     __syncthreads();
-    for (long long s = w0 + threadIdx.x; s < w1; s += POP_NT) {
+#pragma unroll 1
+    for (int s = w0 + threadIdx.x; s < w1; s += POP_NT) {
       const long long p = base + s;
       if (p >= a.capacity) break;
-      const uint32_t c = (uint32_t)(c0 + list[s - w0]);
-      const uint32_t iz = c % n, cy = c / n;
-      const uint32_t iy = cy % n, ix = cy / n;
-      const Philox4 w = rng_block((uint64_t)p, 0, TAG_DISP, a.k0, a.k1);
-      const double shift = (a.psi != nullptr && a.growth != 0.0) ? a.growth * (double)a.psi[c] : 0.0;
-      typedef float f3 __attribute__((ext_vector_type(3), aligned(4)));
-      const f3 f = {wrap_box(((double)ix + 0.5 + tri_offset(w.x)) * a.H, a.box),
-                    wrap_box(((double)iy + 0.5 + tri_offset(w.y)) * a.H, a.box),
-                    wrap_box(((double)iz + 0.5 + tri_offset(w.z)) * a.H + shift, a.box)};
-      *reinterpret_cast<f3*>(a.pos + 3 * p) = f;
+      emit_particle(a, p, (uint32_t)(c0 + list[s - w0]));
     }
     __syncthreads();   // the list is read before the next window overwrites it
   }
 }
-__global__ void __launch_bounds__(POP_NT) k_pop_emit(PopK a) {
-  if (a.rsum[blockIdx.x] == 0.0) pop_emit_body<false>(a, blockIdx.x);
+
+// Windows first, first + step, ... of EMIT_WIN particles of block blk: pre holds every cell's first
+// slot, clipped to the window, and a particle finds its cell by bisection.  SAT: the block holds
+// saturated counts, which are drawn again into LDS (big); in a kernel of its own, since the draws take
+// 132 registers against 60.
+constexpr int EMIT_SPLIT = 16;        // emitting blocks that share the windows of one block
+constexpr int EMIT_DENSE_MAX = 512;   // blocks emitted at a time
+template <bool SAT>
+__device__ __forceinline__ void emit_dense(const PopK& a, int blk, int first, int step, uint16_t* pre, int* big) {
+  __shared__ long long sh[POP_NT / 64];
+  const int tid = threadIdx.x;
+  const int64_t c0 = (int64_t)blk * POP_CELLS;
+  const long long base = a.boff[blk];
+  const ulonglong2 v = load_counts(a, blk);
+  auto stored = [&](int i) { return (int)(((i < 8 ? v.x : v.y) >> (8 * (i & 7))) & 255u); };
+  long long own = 0;
+  if constexpr (SAT) {
+#pragma unroll 1
+    for (int i = 0; i < EMIT_PER; ++i) {
+      int n = stored(i);
+      if (n == 255) {
+        const int64_t c = c0 + tid * EMIT_PER + i;
+        int n0, n1;
+        pair_counts(a, c & ~(int64_t)1, a.misc[0], n0, n1);
+        n = c & 1 ? n1 : n0;
+      }
+      big[i * POP_NT + tid] = n;
+      own += n;
+    }
+  } else {
+    own = bytes_sum(v.x, v.y);
+  }
+  long long total;
+  const long long mine = block_scan_i64<POP_NT>(own, sh, total);
+  for (long long w0 = (long long)first * EMIT_WIN; w0 < total; w0 += (long long)step * EMIT_WIN) {   // block-uniform
+    long long p = mine - w0;
+    uint32_t* out = reinterpret_cast<uint32_t*>(pre) + tid * (EMIT_PER / 2);
+#pragma unroll 1
+    for (int i = 0; i < EMIT_PER; i += 2) {
+      const uint32_t e = (uint32_t)min(max(p, 0ll), (long long)EMIT_WIN);
+      p += SAT ? big[i * POP_NT + tid] : stored(i);
+      const uint32_t o = (uint32_t)min(max(p, 0ll), (long long)EMIT_WIN);
+      p += SAT ? big[(i + 1) * POP_NT + tid] : stored(i + 1);
+      out[i / 2] = e | o << 16;
+    }
+    __syncthreads();
+    const int last = (int)min((long long)EMIT_WIN, total - w0);
+#pragma unroll 1
+    for (int s = tid; s < last; s += POP_NT) {
+      const long long q = base + w0 + s;
+      if (q >= a.capacity) break;
+      int cell = 0;   // the last cell whose first slot is not above s
+#pragma unroll
+      for (int half = POP_CELLS / 2; half > 0; half >>= 1) cell += pre[cell + half] <= s ? half : 0;
+      emit_particle(a, q, (uint32_t)(c0 + cell));
+    }
+    __syncthreads();   // the window's slots are read before the next one's are written
+  }
 }
-__global__ void __launch_bounds__(POP_NT) k_pop_emit_saturated(PopK a) {
-  for (int b = blockIdx.x; b < a.nblk; b += gridDim.x)   // block-uniform
-    if (a.rsum[b] != 0.0) pop_emit_body<true>(a, b);
+// the blocks of one list, dealt over the grid's first nx EMIT_SPLIT blocks: consecutive ones take
+// different dense blocks, so that the few windows of a not very dense one lie on all XCDs
+template <bool SAT>
+__device__ __forceinline__ void emit_dense_blocks(const PopK& a, int bx, int nx, uint16_t* pre, int* big) {
+  const int count = *pop_list_length(a, SAT);
+  for (int d = bx % nx; d < count; d += nx) {   // block-uniform
+    const int blk = *pop_listed(a, SAT, d), first = bx / nx;
+    const long long end = blk + 1 < a.nblk ? a.boff[blk + 1] : reinterpret_cast<const long long*>(a.misc)[1];
+    if ((long long)first * EMIT_WIN < end - a.boff[blk]) emit_dense<SAT>(a, blk, first, EMIT_SPLIT, pre, big);
+  }
+}
+// the first nx EMIT_SPLIT blocks take the dense blocks, the others one sparse block each
+__global__ void __launch_bounds__(POP_NT) k_pop_emit(PopK a, int nx) {
+  __shared__ __align__(16) uint16_t lds[EMIT_WIN > POP_CELLS ? EMIT_WIN : POP_CELLS];
+  const int nd = nx * EMIT_SPLIT, bx = blockIdx.x;
+  if (bx < nd) emit_dense_blocks<false>(a, bx, nx, lds, nullptr);
+  else if (pop_route(a)[bx - nd] == EMIT_SPARSE) emit_sparse(a, bx - nd, lds);
+}
+__global__ void __launch_bounds__(POP_NT) k_pop_emit_saturated(PopK a, int nx) {
+  __shared__ __align__(16) uint16_t pre[POP_CELLS];
+  __shared__ int big[POP_CELLS];
+  emit_dense_blocks<true>(a, blockIdx.x, nx, pre, big);
 }
 
 namespace {
@@ -525,9 +623,9 @@ int populate_place(const float* field, const float* psi, double growth, int n, d
                    void* ws, float* pos, int64_t capacity, hipStream_t s) {
   if (capacity == 0) return PK_OK;
   const PopK a = make_pop(field, psi, n, box, 0.0, bias, growth, seed, ws, nullptr, pos, (long long)capacity);
-  hipLaunchKernelGGL(k_pop_emit, dim3(a.nblk), dim3(POP_NT), 0, s, a);
-  hipLaunchKernelGGL(k_pop_emit_saturated, dim3(a.nblk < EMIT_SAT_BLOCKS ? a.nblk : EMIT_SAT_BLOCKS), dim3(POP_NT), 0,
-                     s, a);
+  const int nx = a.nblk < EMIT_DENSE_MAX ? a.nblk : EMIT_DENSE_MAX;
+  hipLaunchKernelGGL(k_pop_emit, dim3(nx * EMIT_SPLIT + a.nblk), dim3(POP_NT), 0, s, a, nx);
+  hipLaunchKernelGGL(k_pop_emit_saturated, dim3(nx * EMIT_SPLIT), dim3(POP_NT), 0, s, a, nx);
   return check_hip(hipGetLastError(), "population place launch");
 }
 
