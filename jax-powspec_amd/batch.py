@@ -132,8 +132,10 @@ class BatchEstimator:
         self.jobs: list[_Job] = []
         self._table = (_lib.PkJob * self.max_jobs)()
         # graphs cannot capture the legacy default stream: the batch works on its own
-        # stream, ordered after / before the caller's stream with events
+        # stream, ordered after / before the caller's stream with events; and after this one, which
+        # fills the statistics and may still use what the workspace's memory held before
         self._stream = torch.cuda.Stream(device=self.device)
+        self._stream.wait_stream(torch.cuda.current_stream(self.device))
 
     def _on_stream(self, stream, fn):
         cur = stream if stream is not None else torch.cuda.current_stream(self.device)
@@ -157,7 +159,8 @@ class BatchEstimator:
         cats = list(catalogues)
         if len(cats) > self.max_jobs:
             raise ValueError(f"{len(cats)} catalogues exceed the batch capacity {self.max_jobs}")
-        jobs = [c if isinstance(c, _Job) else _Job(c, self.n, self.device) for c in cats]
+        with torch.cuda.stream(stream):   # conversions of the inputs, in the order of the caller's stream
+            jobs = [c if isinstance(c, _Job) else _Job(c, self.n, self.device) for c in cats]
         for i, j in enumerate(jobs):
             if j.np > self.max_particles:
                 raise ValueError(f"catalogue {i}: {j.np} particles exceed the batch capacity {self.max_particles}")

@@ -367,15 +367,14 @@ class Estimator:
                                          device=self.device)
 
     def run(self, x, y, z, w=None, *, stream=None):
-        xs, sx = _device.as_f32_vector(x, self.device, "x")
-        ys, sy = _device.as_f32_vector(y, self.device, "y")
-        zs, sz = _device.as_f32_vector(z, self.device, "z")
+        with torch.cuda.stream(stream):   # conversions of the inputs, in the order of the run's stream
+            xs, sx = _device.as_f32_vector(x, self.device, "x")
+            ys, sy = _device.as_f32_vector(y, self.device, "y")
+            zs, sz = _device.as_f32_vector(z, self.device, "z")
+            ws_, sw = (None, 1) if w is None else _device.as_f32_vector(w, self.device, "w")
         np_ = xs.numel()
         if np_ > self.max_particles:
             raise ValueError(f"{np_} particles exceed the preallocated {self.max_particles}")
-        ws_, sw = (None, 1)
-        if w is not None:
-            ws_, sw = _device.as_f32_vector(w, self.device, "w")
         o = self.out
         _lib.check("pk_estimate", _lib.load().pk_estimate(
             self.plan.handle, _device.ptr(xs), sx, _device.ptr(ys), sy, _device.ptr(zs), sz, _device.ptr(ws_), sw,

@@ -151,6 +151,7 @@ class _PlainEngine:
         self.stats_t = torch.zeros(_lib.STATS_LEN, dtype=torch.float64, device=device)
         self.bytes = need + max_nb * (24 + 8 + 12 + 4 + 8)
         self.stream = torch.cuda.Stream(device=device)
+        self.stream.wait_stream(torch.cuda.current_stream(device))   # the fill of the statistics
         self.busy = None
 
     def fits(self, req):
@@ -160,7 +161,8 @@ class _PlainEngine:
         (f,) = futs
         st = self.stream
         st.wait_event(f.ready)
-        j = _Job(f.req, self.n, self.device)
+        with torch.cuda.stream(st):   # conversions of the inputs, once they are complete
+            j = _Job(f.req, self.n, self.device)
         o = self.out
         with torch.cuda.device(self.device):
             _lib.check("pk_estimate", _lib.load().pk_estimate(
