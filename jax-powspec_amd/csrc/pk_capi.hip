@@ -5,7 +5,9 @@
 #include <stdio.h>
 #include <string.h>
 
+#include <map>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "pk_common.h"
@@ -40,6 +42,20 @@ int num_cus(int device) {
   if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || v < 1) v = 1;
   if (device >= 0 && device < 64) cache[device] = v;
   return v;
+}
+
+int allow_dynamic_lds(const void* kernel, size_t bytes) {
+  static std::mutex mu;
+  static std::map<std::pair<int, const void*>, size_t> allowed;
+  int dev = 0;
+  (void)hipGetDevice(&dev);
+  std::lock_guard<std::mutex> lk(mu);
+  size_t& have = allowed[{dev, kernel}];
+  if (have >= bytes) return PK_OK;
+  const int e = check_hip(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes),
+                          "LDS attribute");
+  if (!e) have = bytes;
+  return e;
 }
 
 // ------------------------------------------------------------------------------------

@@ -1747,20 +1747,13 @@ template <int N> struct FFTLaunch {
     if (m == XB_WIDE) return cmin(g, dyn_cap<XB_WIDE>(nb));
     return g;
   }
-  // raises a kernel's dynamic-LDS limit to its capacity, once (not again inside a capture)
-  template <int M, typename K> static int allow_bins(K kernel, bool& done) {
-    if (done) return PK_OK;
-    const int e = check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                (int)XBin<N, M>::dyn_bytes(XBin<N, M>::CAP)),
-                            "LDS attribute");
-    done = e == PK_OK;
-    return e;
+  // raises a kernel's dynamic-LDS limit to its capacity
+  template <int M, typename K> static int allow_bins(K kernel) {
+    return allow_dynamic_lds(reinterpret_cast<const void*>(kernel), XBin<N, M>::dyn_bytes(XBin<N, M>::CAP));
   }
   template <int M> static int launch_bin(const Job& j, const float2* tw, int grid, hipStream_t s) {
     if constexpr (M >= XB_TALL) {
-      static bool done = false;
-      const int e = allow_bins<M>(k_xpass_bin<N, M>, done);
+      const int e = allow_bins<M>(k_xpass_bin<N, M>);
       if (e) return e;
     }
     hipLaunchKernelGGL((k_xpass_bin<N, M>), dim3(grid), dim3(XBin<N, M>::NT), (XBin<N, M>::dyn_bytes(j.nb)), s, j,
@@ -1770,8 +1763,7 @@ template <int N> struct FFTLaunch {
   template <int M>
   static int launch_bin_jobs(const Job* jobs, int njobs, int max_nb, int gx, const float2* tw, hipStream_t s) {
     if constexpr (M >= XB_TALL) {
-      static bool done = false;
-      const int e = allow_bins<M>(k_xpass_bin_jobs<N, M>, done);
+      const int e = allow_bins<M>(k_xpass_bin_jobs<N, M>);
       if (e) return e;
     }
     hipLaunchKernelGGL((k_xpass_bin_jobs<N, M>), dim3(gx, njobs), dim3(XBin<N, M>::NT),

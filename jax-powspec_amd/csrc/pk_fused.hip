@@ -290,10 +290,7 @@ template <int N, int TY> struct FusedLaunch {
   static bool ok(const TileGeom& g) { return g.ty == TY && Cf::LDS + Cf::STATIC_LDS <= 160 * 1024; }
   template <typename K>
   static int attr(K k) {
-    if (Cf::LDS <= 65536) return PK_OK;
-    return check_hip(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                         (int)Cf::LDS),
-                     "LDS attribute");
+    return Cf::LDS <= 65536 ? PK_OK : allow_dynamic_lds(reinterpret_cast<const void*>(k), Cf::LDS);
   }
   // persistent grid: resident blocks of the whole GPU (LDS-limited), at most one per tile
   static int grid() {
@@ -312,12 +309,8 @@ template <int N, int TY> struct FusedLaunch {
   }
   template <int ST>
   static int run_st(const Job& j, const float2* tw, hipStream_t s) {
-    static bool done = false;
-    if (!done) {
-      int e = attr(k_fused_deposit_zpass<N, TY, ST>);
-      if (e) return e;
-      done = true;
-    }
+    const int e = attr(k_fused_deposit_zpass<N, TY, ST>);
+    if (e) return e;
     const int gx = j.g.ntiles < grid() ? j.g.ntiles : grid();
     StageTimer t(ST_DEPOSIT, s);
     hipLaunchKernelGGL((k_fused_deposit_zpass<N, TY, ST>), dim3(gx), dim3(Cf::NT), Cf::LDS, s, j, tw);
@@ -329,12 +322,8 @@ template <int N, int TY> struct FusedLaunch {
     return run_st<PK_STENCIL_TSC>(j, tw, s);
   }
   static int run_jobs(const Job* jobs, int njobs, int ntiles, const float2* tw, hipStream_t s) {
-    static bool done = false;
-    if (!done) {
-      int e = attr(k_fused_deposit_zpass_jobs<N, TY>);
-      if (e) return e;
-      done = true;
-    }
+    const int e = attr(k_fused_deposit_zpass_jobs<N, TY>);
+    if (e) return e;
     // one block per tile: jobs of very different sizes share the launch, and dynamic block
     // scheduling balances them better than a fixed share of a persistent grid per job
     const int gx = ntiles;

@@ -7,6 +7,9 @@
 namespace pk {
 
 int num_cus(int device);
+// Raises a kernel's dynamic-LDS limit on the current device, which has limits of its own: once per device
+// and size (not again inside a graph capture).
+int allow_dynamic_lds(const void* kernel, size_t bytes);
 
 // ---- mass assignment (pk_scatter.hip) -----------------------------------------------
 struct ScatterArgs {

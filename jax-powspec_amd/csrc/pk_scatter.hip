@@ -24,10 +24,6 @@
 //              writes each row once with coalesced stores: no global atomics, no zero fill.
 //   5. atomic: the (normally empty) irregular bucket is added with global atomics.
 // A direct mode (tile[0] == 0) adds every particle with global atomics instead.
-#include <mutex>
-#include <utility>
-#include <vector>
-
 #include "pk_particles.h"
 
 namespace pk {
@@ -895,19 +891,8 @@ int grid_for(int64_t items, int nt, int cap) {
   return (int)gsz;
 }
 
-// raises a kernel's dynamic-LDS limit once per size (not again inside a graph capture)
-template <typename K>
-int allow_lds(K kernel, size_t bytes) {
-  if (bytes <= 65536) return PK_OK;
-  static std::mutex mu;
-  static std::vector<std::pair<const void*, size_t>> done;
-  const void* k = reinterpret_cast<const void*>(kernel);
-  std::lock_guard<std::mutex> lk(mu);
-  for (auto& d : done)
-    if (d.first == k && d.second >= bytes) return PK_OK;
-  int e = check_hip(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes), "LDS attribute");
-  if (!e) done.emplace_back(k, bytes);
-  return e;
+template <typename K> int allow_lds(K kernel, size_t bytes) {
+  return bytes <= 65536 ? PK_OK : allow_dynamic_lds(reinterpret_cast<const void*>(kernel), bytes);
 }
 
 size_t hist_lds(const TileGeom& g, int n) {
