@@ -686,7 +686,7 @@ SlotLayout slot_layout(int n, int64_t max_np, int max_nb, const TileGeom& cap, i
   cj.g = cap;
   cj.a.n = n;
   cj.a.np = max_np;
-  off += carve_scatter(cj, false, nullptr);
+  off += carve_scatter(cj, false, batch_sort_scratch(cap, n), nullptr);
   L.bytes = align_up(off);
   return L;
 }
@@ -762,7 +762,7 @@ int pk_batch_create(pk_plan* p, int max_jobs, int64_t max_np, int max_nb, const 
     j.a.np = max_np;
     j.spec = reinterpret_cast<float2*>(base + L.spec);
     j.partials = reinterpret_cast<double*>(base + L.partials);
-    carve_scatter(j, false, base + L.scatter);   // also points j.stats at the slot's own stats
+    carve_scatter(j, false, batch_sort_scratch(b->cap, p->n), base + L.scatter);   // also points j.stats at the slot's own stats
   }
   for (int k = 0; k < 2; ++k) {
     b->h_jobs[k] = nullptr;

@@ -48,6 +48,13 @@ __host__ __device__ inline int count_columns(const TileGeom& g, int n) {
   return g.sort == SORT_PLANES ? n + 1 : g.nkeys;
 }
 __host__ __device__ inline int group_count(const TileGeom& g, int n) { return g.sort == SORT_KEYS ? g.nkeys : n + 1; }
+// what a sort keeps in its scratch beyond what every one keeps
+struct SortScratch {
+  int columns;   // of the count matrix
+  bool mixed;    // the x planes' counts beside the keys'
+  bool planes;   // the planes' starts
+  bool staged;   // the records grouped by x plane only
+};
 
 // LDS bytes up to which the deposit accumulates in 64-bit fixed point: gfx950 LDS
 // integer atomics run ~13x faster than float ones, and integer sums are order-independent
@@ -159,8 +166,11 @@ int sort_column_blocks(const TileGeom& g, int n);
 // particles per counting block (clamped to the supported range) and the block count
 void set_chunk(TileGeom* g, int64_t np, int64_t chunk);
 size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int n, int64_t np);
+SortScratch sort_scratch(const TileGeom& g, int n);
+// scratch of every sort that the jobs of a batch of geometry cap (its most classes) may take
+SortScratch batch_sort_scratch(const TileGeom& cap, int n);
 // points the sorted-deposit scratch of j into base (nullptr: sizes only); returns bytes
-size_t carve_scatter(Job& j, bool direct, void* base);
+size_t carve_scatter(Job& j, bool direct, const SortScratch& need, void* base);
 // mesh_out == nullptr (tiled mode only): stop after sorting; the caller runs the fused
 // deposit + z pass on j's sorted records
 int scatter_run(Job& j, bool direct, const float* mesh_in, float* mesh_out, void* ws, size_t ws_bytes,

@@ -826,6 +826,27 @@ static int largest_divisor_le(int n, int cap) {
   return n;
 }
 
+static int sort_of(long nkeys) {
+  return nkeys <= SORT_KEYS_MAX ? SORT_KEYS : nkeys <= COUNT_KEYS_MAX ? SORT_MIXED : SORT_PLANES;
+}
+
+SortScratch sort_scratch(const TileGeom& g, int n) {
+  return {count_columns(g, n), g.sort == SORT_MIXED, g.sort == SORT_PLANES, g.sort != SORT_KEYS};
+}
+
+SortScratch batch_sort_scratch(const TileGeom& cap, int n) {
+  SortScratch r = sort_scratch(cap, n);
+  for (int ncls = 2; ncls < cap.ncls; ++ncls) {
+    TileGeom g = cap;
+    g.ncls = ncls;
+    g.nkeys = cap.ntiles * ncls + 1;
+    g.sort = sort_of(g.nkeys);
+    const SortScratch s = sort_scratch(g, n);
+    r = {s.columns > r.columns ? s.columns : r.columns, r.mixed || s.mixed, r.planes || s.planes, r.staged || s.staged};
+  }
+  return r;
+}
+
 void set_chunk(TileGeom* g, int64_t np, int64_t chunk) {
   if (chunk < CHUNK_MIN) chunk = CHUNK_MIN;
   if (chunk > CHUNK_MAX) chunk = CHUNK_MAX;
@@ -871,7 +892,7 @@ int make_tile_geom(int n, int64_t np, int stencil, const int* tile, TileGeom* g,
   g->ntiles = (int)ntiles;
   g->nkeys = (int)nkeys;
   g->fixed = (size_t)ty * n * 8 <= FIXED_LDS_MAX ? 1 : 0;
-  g->sort = nkeys <= SORT_KEYS_MAX ? SORT_KEYS : nkeys <= COUNT_KEYS_MAX ? SORT_MIXED : SORT_PLANES;
+  g->sort = sort_of(nkeys);
   // one counting / placing block per CU when the catalogue is large (a second, partial
   // round of blocks would cost a whole round), at least CHUNK_MIN particles per block
   int dev = 0;
@@ -905,7 +926,7 @@ size_t plane_keys_lds(const TileGeom& g) { return (size_t)g.nyt * g.ncls * sizeo
 
 int sort_column_blocks(const TileGeom& g, int n) { return column_blocks(g, n); }
 
-size_t carve_scatter(Job& j, bool direct, void* base) {
+size_t carve_scatter(Job& j, bool direct, const SortScratch& need, void* base) {
   size_t off = 0;
   char* b = static_cast<char*>(base);
   auto take = [&](size_t bytes) -> void* {
@@ -917,18 +938,19 @@ size_t carve_scatter(Job& j, bool direct, void* base) {
   double* st = static_cast<double*>(take(PK_STATS_LEN * sizeof(double)));
   if (!j.stats) j.stats = st;
   if (!direct) {
-    j.mat = static_cast<unsigned*>(take((size_t)g.nblk * g.nkeys * sizeof(unsigned)));
-    j.pmat = static_cast<unsigned*>(take((size_t)g.nblk * (j.a.n + 1) * sizeof(unsigned)));
-    j.totals = static_cast<int*>(take((size_t)g.nkeys * sizeof(int)));
-    j.ptotals = static_cast<int*>(take(((size_t)j.a.n + 1) * sizeof(int)));
+    const size_t planes = (size_t)j.a.n + 1;   // and the irregular key
+    j.mat = static_cast<unsigned*>(take((size_t)g.nblk * need.columns * sizeof(unsigned)));
+    j.pmat = static_cast<unsigned*>(take(need.mixed ? g.nblk * planes * sizeof(unsigned) : 0));
+    j.totals = static_cast<int*>(take((size_t)need.columns * sizeof(int)));
+    j.ptotals = static_cast<int*>(take(need.mixed ? planes * sizeof(int) : 0));
     j.key_start = static_cast<int*>(take(((size_t)g.nkeys + 1) * sizeof(int)));
-    j.plane_start = static_cast<int*>(take(((size_t)j.a.n + 2) * sizeof(int)));
+    j.plane_start = static_cast<int*>(take(need.planes ? (planes + 1) * sizeof(int) : 0));
     j.wsum = static_cast<double*>(take((size_t)g.nblk * sizeof(double)));
     j.wmax = static_cast<double*>(take((size_t)g.nblk * sizeof(double)));
     j.aux = static_cast<double*>(take(AUX_LEN * sizeof(double)));
     j.koff = static_cast<unsigned*>(take((size_t)g.nkeys * sizeof(unsigned)));
     j.sorted = take((size_t)(j.a.np > 0 ? j.a.np : 1) * sizeof(float4));
-    j.staged = take((size_t)(j.a.np > 0 ? j.a.np : 1) * sizeof(float4));
+    j.staged = take(need.staged ? (size_t)(j.a.np > 0 ? j.a.np : 1) * sizeof(float4) : 0);
     j.tile_mass = static_cast<double*>(take((size_t)g.ntiles * sizeof(double)));
     j.tile_sq = static_cast<double*>(take((size_t)g.ntiles * sizeof(double)));
   }
@@ -940,7 +962,7 @@ size_t scatter_workspace_bytes(const TileGeom& g, bool direct, int n, int64_t np
   j.g = g;
   j.a.np = np;
   j.a.n = n;
-  return carve_scatter(j, direct, nullptr);
+  return carve_scatter(j, direct, sort_scratch(g, n), nullptr);
 }
 
 int mass_finalize(const Job& j, hipStream_t s) {
@@ -951,7 +973,7 @@ int mass_finalize(const Job& j, hipStream_t s) {
 
 int scatter_run(Job& j, bool direct, const float* mesh_in, float* mesh_out, void* ws, size_t ws_bytes,
                 hipStream_t s) {
-  const size_t need = carve_scatter(j, direct, ws);
+  const size_t need = carve_scatter(j, direct, sort_scratch(j.g, j.a.n), ws);
   if (ws_bytes < need) return set_error(PK_E_WORKSPACE, "scatter workspace %zu < %zu bytes", ws_bytes, need);
   const ScatterArgs& a = j.a;
   const TileGeom& g = j.g;

@@ -4,22 +4,22 @@ import os
 import subprocess
 import sys
 
-import pytest
-
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 
-PROGRAM = """
-import ctypes as C, sys
+PRELUDE = """
+import ctypes as C, sys, types
 fake = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
-sys.path.insert(0, sys.argv[2])
-import types
-pkg = types.ModuleType("jax_powspec_amd"); pkg.__path__ = [sys.argv[2] + "/jax-powspec_amd"]
+pkg = types.ModuleType("jax_powspec_amd")
+pkg.__path__ = [sys.argv[2] + "/jax-powspec_amd"]
 sys.modules["jax_powspec_amd"] = pkg
 from jax_powspec_amd import _lib
 lib = _lib.load()
 P = 4096                     # stands for every device pointer; nothing reads it
 ok = lambda r: r == 0 or sys.exit(lib.pk_last_error())
+"""
+
+PROGRAM = """
 def run(device, n, nb, stencil):
     fake.fake_set_device(device)
     plan, need = C.c_void_p(), C.c_size_t()
@@ -48,18 +48,21 @@ for device in (0, 1, 0, 1):
 """
 
 
-@pytest.fixture(scope="module")
-def log(tmp_path_factory):
-    lib = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+
+
+def lines_of(program, folder):
+    """what a program prints that runs after PRELUDE"""
+    lib = str(folder / "libfake_hip.so")
     subprocess.run(["g++", "-O1", "-shared", "-fPIC", os.path.join(HERE, "fake_hip.cpp"), "-o", lib], check=True)
-    r = subprocess.run([sys.executable, "-c", PROGRAM, lib, ROOT], capture_output=True, text=True, timeout=60)
+    r = subprocess.run([sys.executable, "-c", PRELUDE + program, lib, ROOT], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stderr
-    return [line.split(" ", 3) for line in r.stdout.splitlines()]
+    return r.stdout.splitlines()
 
 
-def test_every_device_raises_the_limits(log):
+def test_every_device_raises_the_limits(tmp_path):
     limit, launches = {}, 0
-    for what, device, value, kernel in log:
+    for line in lines_of(PROGRAM, tmp_path):
+        what, device, value, kernel = line.split(" ", 3)
         if what == "attribute":
             assert int(value) > limit.get((device, kernel), 0), f"set again: {kernel}"
             limit[device, kernel] = int(value)
