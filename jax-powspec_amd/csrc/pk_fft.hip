@@ -932,6 +932,8 @@ k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__
     {
       float2 v[F::PER0][F::R0];
       F::each_first(to, [&](int t, int r, int row, int c) { v[t][r] = base[row * N + c]; });
+      // the contrast's modes: squares of the density's leave float's range for large and small weights
+      F::each_first(to, [&](int t, int r, int, int) { v[t][r] = make_float2(sf * v[t][r].x, sf * v[t][r].y); });
       F::first(to, v, buf);
     }
     // the factors of the modes this thread will hold, while no transform values occupy its
@@ -956,7 +958,7 @@ k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__
             g = wt[row] * wt[y] * wz * (coef(3 * slot) + coef(3 * slot + 1) * l2 + coef(3 * slot + 2) * l4);
           }
         }
-        sc[t][r] = 2.0f * g * sf;
+        sc[t][r] = 2.0f * g;
         __builtin_amdgcn_sched_barrier(0);
       });
     }
@@ -982,7 +984,7 @@ k_xpass_adjoint(Job j, const float2* __restrict__ twg, const float* __restrict__
     }
     __syncthreads();   // the tile is read before the next one's first stage overwrites it
   }
-  const double t = block_sum_f64_waves<NT>(acc * (double)sf, red);
+  const double t = block_sum_f64_waves<NT>(acc, red);
   if (tid == 0) gsum_part[blockIdx.x] = t;
 }
 
