@@ -85,14 +85,16 @@ def upload(a, device: torch.device) -> torch.Tensor:
     capture the copy stays a pageable one, which the capture refuses: a replay would read a
     pinned block that has gone to another use.)
     """
+    if device.index != torch.cuda.current_device():   # that device's stream takes the copy: its capture counts
+        with torch.cuda.device(device):
+            return upload(a, device)
     src = torch.from_numpy(np.ascontiguousarray(a))
-    with torch.cuda.device(device):   # whose stream takes the copy: a capture of that one counts
-        if torch.cuda.is_current_stream_capturing():
-            return src.to(device)
-        # on the host by name: torch.set_default_device moves what is made without a device
-        pinned = torch.empty(src.shape, dtype=src.dtype, device="cpu", pin_memory=True)
-        pinned.copy_(src)
-        return pinned.to(device, non_blocking=True)
+    if torch.cuda.is_current_stream_capturing():
+        return src.to(device)
+    # on the host by name: torch.set_default_device moves what is made without a device
+    pinned = torch.empty(src.shape, dtype=src.dtype, device="cpu", pin_memory=True)
+    pinned.copy_(src)
+    return pinned.to(device, non_blocking=True)
 
 
 def as_f32_vector(a, device: torch.device, name: str) -> tuple[torch.Tensor, int]:
