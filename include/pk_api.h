@@ -99,7 +99,12 @@ int pk_supported_n(int n);   /* 1 if n is supported, else 0 */
  * LDS-privatised deposit (ty rows of full z extent; tile[2] may be 0 for n); tile == NULL
  * picks the default (ty = largest divisor of n that is <= 32 and keeps ty n 8 bytes within
  * 128 KB: 32 up to n = 512, 16 at 768 and 1024); tile[0] == 0 selects direct global
- * atomics.  Every n uses the sorted deposit unless direct is asked for.  stats (nullable) receives the deposited mass (PK_STATS_LEN doubles).
+ * atomics, whose float sums depend on the order of the adds.  With tile == NULL every n takes the
+ * sorted, order-independent deposit but odd n above 127 without a divisor whose rows fit (131, 257,
+ * 1369: primes, products of large primes), which take global atomics.  In the sorted deposit, too,
+ * particles that the reference stencil treats as out of range (base index outside the mesh, or two
+ * coordinates left of it) are added to a mesh with global atomics.  stats (nullable) receives the
+ * deposited mass (PK_STATS_LEN doubles).
  * Index/fraction arithmetic follows the reference in float32: inv = 1 / ((float)box /
  * (float)n), pos = (x - xmin) * inv.
  */

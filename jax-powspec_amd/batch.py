@@ -208,8 +208,8 @@ class BatchEstimator:
         return self
 
     def _centres(self, indices):
-        """Bin centres (float32, device) of the jobs whose edges were given, in one copy; None for
-        fundamental bins."""
+        """{index: bin centres (float32, device)} of the jobs whose edges were given, sent in one copy;
+        jobs with fundamental bins have no entry."""
         host = {i: (0.5 * (j.edges[1:] + j.edges[:-1]) * (2.0 * np.pi / j.box)).astype(np.float32)
                 for i, j in ((i, self.jobs[i]) for i in indices) if not j.fundamental}
         if not host:

@@ -116,8 +116,11 @@ template <> struct DFT<8> {
 // ------------------------------------------------------------------------------------
 // radix plan: as many 8s as possible, then 6 (where it ends the plan), 4, 2, 3.  The 6 saves the
 // passes at 384 one of four stages (8 8 6 for 8 8 2 3): estimate 473 -> 459 us (TSC, 3e6 particles),
-// xi_vec 470 -> 429 us, estimate_ad 1177 -> 1092 us.  Error of P_l against 64 bits, rms over the bins:
-// 9.8e-8 -> 8.2e-8 at 48 (40 meshes), 1.05e-7 -> 9.7e-8 at 96 (24), 1.07e-7 -> 1.04e-7 at 384 (10).
+// xi_vec 470 -> 429 us, estimate_ad 1177 -> 1092 us.  Error against 64 bits in the 2-norm over the bins
+// (led by the few low-k ones), mean over meshes: P_l at 48 9.3e-8 -> 8.0e-8 (150 meshes), estimates there
+// 9.7e-8 -> 8.2e-8 (150), xi 2.16e-7 -> 1.68e-7 (100), 96 1.36e-7 -> 1.34e-7 (80), 384 1.7e-7 -> 1.2e-7 (10);
+// each bin weighed the same, 9.8e-8 -> 8.2e-8 at 48 (40), 1.05e-7 -> 9.7e-8 at 96 (24), 1.07e-7 -> 1.04e-7 at
+// 384 (10).
 // ------------------------------------------------------------------------------------
 __host__ __device__ constexpr int radix_next(int m) {
   return (m % 8 == 0) ? 8 : m == 6 ? 6 : (m % 4 == 0) ? 4 : (m % 2 == 0) ? 2 : (m % 3 == 0) ? 3 : 1;

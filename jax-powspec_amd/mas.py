@@ -96,7 +96,9 @@ def assign(x, y, z, w=None, *, box_size, n_bins, mas="CIC_REF", wrap=True, xmin=
     mas: 'CIC_REF' (reference stencil, cic_mas_vec), 'CIC' (textbook, mass-conserving,
     periodic) or 'TSC'.  delta: optional accumulation base (None = zeros).
     tile: (1, ty, 0) row-bundle tile of the sorted deposit (ty rows of full z extent, ty | n),
-          'direct' for global atomics, or None (ty = largest divisor of n <= 32).
+          'direct' for global atomics (float sums in any order), or None: ty = the largest divisor
+          of n up to 32 whose rows fit 128 KB of 64-bit cells, and n itself where no divisor is in
+          that range and they fit; odd n above 127 without either (131, 257, 1369) take global atomics.
     stats: optional float64 device tensor of 4 entries receiving [mass, n^3/mass, -, -].
     """
     mas = mas.upper()
