@@ -56,10 +56,9 @@ template <int N, int TY_> struct FusedCfg {
   static constexpr int WPE = cmax(1, cmin(4, cmax(1, BPC) * (NT / 64) / 4));
 };
 
-// Deposits are rint(W w S) with S = 2^(30 - e), max |w| < 2^e and corner weights W <= 1, so
-// each is below 2^30 and converts through int32; a cell of R records sums below R 2^30 and a
-// tile's cells below 9 R 2^30, inside int64 for any catalogue of < 2^29 particles (irregular
-// records: W <= 8, converted in 64 bits).  The
+// Deposits are rint(W w S) with S = 2^(30 - e), max |w| corner_weight_bound < 2^e, so each is
+// below 2^30 (2^31 at one negative coordinate) and converts through int32; a cell of R records sums
+// below R 2^30 and a tile's cells below 9 R 2^30, inside int64 for any catalogue of < 2^29 particles.  The
 // quantum 2^(e - 30) must stay this fine: the rounding is white noise on the mesh, and it
 // enters |delta_k|^2 through the cross term with the signal, i.e. as the square root of its
 // power, which the TSC window's deconvolution at the corner of the spectrum exposes
@@ -153,15 +152,10 @@ __device__ __forceinline__ void fused_body(const Job& j, int bx, int nbx, const 
       const int ly = iy - y0;
       if ((unsigned)ly < (unsigned)C) atomicAdd(&acc[iz * C + ly], to_fixed(wt));
     };
-    auto add_wide = [&](int iy, int iz, float wt) {
-      const int ly = iy - y0;
-      if ((unsigned)ly < (unsigned)C) atomicAdd(&acc[iz * C + ly], to_fixed_wide(wt));
-    };
     auto dep = [&](const float4& r, bool reg) {
       const float ws = record_weight(r, has_w) * scale;
-      if (stencil != PK_STENCIL_CIC_REF) for_each_corner_on_x<ST>(a, r.x, r.y, r.z, ws, xt, add);
-      else if (reg) ref_corners_on_x_regular(a, r.x, r.y, r.z, ws, xt, add);
-      else for_each_corner_on_x<PK_STENCIL_CIC_REF>(a, r.x, r.y, r.z, ws, xt, add_wide);
+      if (stencil == PK_STENCIL_CIC_REF && reg) ref_corners_on_x_regular(a, r.x, r.y, r.z, ws, xt, add);
+      else for_each_corner_on_x<ST>(a, r.x, r.y, r.z, ws, xt, add);
     };
     const int total = B.pre[B.nbk];
 #pragma unroll

@@ -344,21 +344,11 @@ __device__ __forceinline__ int row_key_in_plane(const ScatterArgs& a, const Tile
   return yt * g.ncls + cls;
 }
 
-// Particles of the reference stencil that need its general corners: a truncated base index outside
-// [0, n) on any axis (at or below -1 cell, at or above n) follows the per-corner JAX index rules;
-// and two negative coordinates make corner weights above 2, since truncation towards zero leaves
-// 1 - dd in (1, 2) there, which the regular records' 32-bit conversion does not hold.
-__device__ __forceinline__ bool ref_irregular(float px, float py, float pz, int n) {
-  const int ix = (int)px, iy = (int)py, iz = (int)pz;
-  return (unsigned)ix >= (unsigned)n || (unsigned)iy >= (unsigned)n || (unsigned)iz >= (unsigned)n ||
-         __builtin_amdgcn_fmed3f(px, py, pz) < 0.0f;
-}
-
 // Row-bundle tiles: tile (xt, yt) owns cells x = xt, y in [yt*ty, yt*ty + ty), all z.
 // Key = tile * ncls + y-class, where the y-class marks the tile rows whose stencil spills
 // into the neighbouring tile (CIC variants: 1 = last row; TSC: 1 = first, 2 = last row).
 // The x neighbours are read whole (one x-layer per tile).  Last key: irregular particles
-// (ref_irregular); -1: dropped.
+// (reference stencil with an out-of-range base index); -1: dropped.
 // plane (optional): the key's x plane hx, or n for the irregular key (keys are x-plane major).
 // ST >= 0 fixes the stencil at compile time (the run-time a.stencil is then ignored).
 template <int ST = -1>
@@ -368,7 +358,10 @@ __device__ __forceinline__ int row_tile_key(const ScatterArgs& a, const TileGeom
   const int n = a.n;
   const int stencil = ST >= 0 ? ST : a.stencil;
   if (stencil == PK_STENCIL_CIC_REF) {
-    if (ref_irregular(px, py, pz, n)) {
+    // irregular: a truncated base index outside [0, n) on any axis (positions below -1 cell
+    // or at or above n), whose corners need the per-corner JAX index rules
+    const int ix = (int)px, iy = (int)py, iz = (int)pz;
+    if ((unsigned)ix >= (unsigned)n || (unsigned)iy >= (unsigned)n || (unsigned)iz >= (unsigned)n) {
       if (plane) *plane = n;
       return g.nkeys - 1;
     }
@@ -385,7 +378,10 @@ __device__ __forceinline__ int row_plane(const ScatterArgs& a, float px, float p
   if (!pos_ok(px, py, pz)) return -1;
   const int n = a.n;
   const int stencil = ST >= 0 ? ST : a.stencil;
-  if (stencil == PK_STENCIL_CIC_REF && ref_irregular(px, py, pz, n)) return n;
+  if (stencil == PK_STENCIL_CIC_REF) {
+    const int ix = (int)px, iy = (int)py, iz = (int)pz;
+    if ((unsigned)ix >= (unsigned)n || (unsigned)iy >= (unsigned)n || (unsigned)iz >= (unsigned)n) return n;
+  }
   return home_cell(px, n, stencil);
 }
 
@@ -467,17 +463,23 @@ __device__ __forceinline__ float4 bucket_record(const TileBuckets& B, const void
   return load_record_stream(sorted, (size_t)B.base[b] + (i - B.pre[b]), has_w);
 }
 
+// Half or more of the largest corner weight of a particle, at most 8.  Corner weights are <= 1, but
+// the reference stencil's truncation towards zero leaves 1 - dd in (1, 2) at a negative coordinate:
+// up to 2, 4 or 8 with one, two or three of them.  (One fits the conversion below as it is.  The count
+// tests it: a conversion in 64 bits for such records in the mesh deposit took 1% of a call at 512^3.)
+template <int ST = -1>
+__device__ __forceinline__ float corner_weight_bound(const ScatterArgs& a, float px, float py, float pz) {
+  const int stencil = ST >= 0 ? ST : a.stencil;
+  return stencil == PK_STENCIL_CIC_REF && __builtin_amdgcn_fmed3f(px, py, pz) < 0.0f ? 8.0f : 1.0f;
+}
+
 // 64-bit fixed-point deposit value (two's complement) of a weight already multiplied by
-// the scale S = 2^(30 - e) with 2^e > max|w|: every corner weight of a regular record is < 2
-// (<= 1 but for the reference stencil at a negative coordinate), so |v| < 2^31, rint(v) fits an
-// int32 and the conversion is one round and one convert (a float -> int64 conversion would take
-// ten instructions per corner).
+// the scale S = 2^(30 - e) with 2^e > max |w| corner_weight_bound: |v| < 2^30, or 2^31 at one negative
+// coordinate, so rint(v) fits an int32 and the conversion is one round and one convert (a float ->
+// int64 conversion would take ten instructions per corner).
 __device__ __forceinline__ unsigned long long to_fixed(float v) {
   return (unsigned long long)(long long)(int)__builtin_rintf(v);
 }
-// irregular records: corner weights up to 8
-__device__ __forceinline__ unsigned long long to_fixed_wide(float v) {
-  return (unsigned long long)(long long)__builtin_rintf(v);
-}
+__device__ __forceinline__ unsigned long long to_fixed(float wt, float scale) { return to_fixed(wt * scale); }
 
 }  // namespace pk

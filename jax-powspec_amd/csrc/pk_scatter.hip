@@ -103,7 +103,7 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
         if (packed) atomicAdd(&hist[key >> 1], 1u << (16 * (key & 1)));
         else atomicAdd(&hist[key], 1u);
         ws += (double)w[u];
-        wm = fmaxf(wm, fabsf(w[u]));
+        wm = fmaxf(wm, fabsf(w[u]) * corner_weight_bound<ST>(a, px[u], py[u], pz[u]));
       }
     }
   }
@@ -215,8 +215,8 @@ __device__ __forceinline__ void weight_stats_body(const Job& j) {
   if (threadIdx.x == 0) {
     const double n = (double)j.a.n;
     j.stats[3] = t / (n * n * n);
-    // fixed-point scale S = 2^30 / 2^e with max|w| < 2^e: every deposit |rint(w W S)| < 2^30
-    // for corner weights W <= 1, so it converts through int32
+    // fixed-point scale S = 2^30 / 2^e, max |w| times the particle's corner_weight_bound < 2^e: every
+    // deposit |rint(w W S)| < 2^31, so it converts through int32
     int e = 0;
     const double wmax = __longlong_as_double((long long)wmax_bits);
     if (wmax > 0.0 && wmax < 1e300) (void)frexp(wmax, &e);
