@@ -454,9 +454,9 @@ __device__ __forceinline__ ulonglong2 load_counts(const PopK& a, int blk) {
 // up its block once they are many (64^3 cells of 40 particles: 1112 us, against 225 to mark the slots
 // from the waves and 84 to emit), so blocks with more than EMIT_OWN in the cells of one thread go by
 // bisection (119 us there).  Whole calls, us, marking / listing alone / both ways as here:
-// 64^3 cells of 40: 395 / 1228 / 208; of 300: 2346 / 35700 / 1234; 128^3, 1 per cell, bias 2: 146 /
-// 215 / 129; 256^3 of 2: 563 / 470 / 457 (EMIT_OWN 32: 514); 256^3 of 0.15: 175 / 139 / 126.  At 512^3
-// with 2e7 particles marking and emitting take 407 + 158 us, this 253 + 4.
+// 64^3 cells of 40: 395 / 1226 / 208; of 300: 2346 / 36000 / 1233; 128^3, 1 per cell, bias 2: 147 /
+// 216 / 130; 256^3 of 2: 565 / 473 / 447 (EMIT_OWN 32: 514); 256^3 of 0.15: 175 / 140 / 124; 64^3 of a half:
+// 54 / 64 / 58.  At 512^3 with 2e7 particles marking and emitting take 407 + 158 us, this 251 + 4.
 // Sparse blocks: a thread scans its 16 cells' counts (one 16-byte load), the block scans the threads'
 // sums, every thread lists its particles' cells in LDS (EMIT_WIN slots at a time), and the lanes then
 // take consecutive particles.
@@ -556,7 +556,7 @@ __device__ __forceinline__ void emit_dense(const PopK& a, int blk, int first, in
     __syncthreads();   // the window's slots are read before the next one's are written
   }
 }
-// the blocks of one list, dealt over the grid's first nx EMIT_SPLIT blocks: consecutive ones take
+// the blocks of one list, dealt over nx EMIT_SPLIT emitting blocks: consecutive ones take
 // different dense blocks, so that the few windows of a not very dense one lie on all XCDs
 template <bool SAT>
 __device__ __forceinline__ void emit_dense_blocks(const PopK& a, int bx, int nx, uint16_t* pre, int* big) {
@@ -567,12 +567,13 @@ __device__ __forceinline__ void emit_dense_blocks(const PopK& a, int bx, int nx,
     if ((long long)first * EMIT_WIN < end - a.boff[blk]) emit_dense<SAT>(a, blk, first, EMIT_SPLIT, pre, big);
   }
 }
-// the first nx EMIT_SPLIT blocks take the dense blocks, the others one sparse block each
+// one sparse block each, then the nx EMIT_SPLIT blocks that take the dense ones (those first, the idle ones
+// of them held the sparse blocks up: 128^3 of 1 42 against 33 us, 256^3 of 2 324 against 309)
 __global__ void __launch_bounds__(POP_NT) k_pop_emit(PopK a, int nx) {
   __shared__ __align__(16) uint16_t lds[EMIT_WIN > POP_CELLS ? EMIT_WIN : POP_CELLS];
-  const int nd = nx * EMIT_SPLIT, bx = blockIdx.x;
-  if (bx < nd) emit_dense_blocks<false>(a, bx, nx, lds, nullptr);
-  else if (pop_route(a)[bx - nd] == EMIT_SPARSE) emit_sparse(a, bx - nd, lds);
+  const int bx = blockIdx.x;
+  if (bx >= a.nblk) emit_dense_blocks<false>(a, bx - a.nblk, nx, lds, nullptr);
+  else if (pop_route(a)[bx] == EMIT_SPARSE) emit_sparse(a, bx, lds);
 }
 __global__ void __launch_bounds__(POP_NT) k_pop_emit_saturated(PopK a, int nx) {
   __shared__ __align__(16) uint16_t pre[POP_CELLS];
