@@ -220,6 +220,7 @@ __device__ __forceinline__ void weight_stats_body(const Job& j) {
     int e = 0;
     const double wmax = __longlong_as_double((long long)wmax_bits);
     if (wmax > 0.0 && wmax < 1e300) (void)frexp(wmax, &e);
+    if (e < -96) e = -96;   // S is used in float
     j.aux[0] = ldexp(1.0, 30 - e);
     j.aux[1] = ldexp(1.0, e - 30);
   }
