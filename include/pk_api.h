@@ -102,9 +102,9 @@ int pk_supported_n(int n);   /* 1 if n is supported, else 0 */
  * atomics, whose float sums depend on the order of the adds.  With tile == NULL every n takes the
  * sorted, order-independent deposit but odd n above 127 without a divisor whose rows fit (131, 257,
  * 1369: primes, products of large primes), which take global atomics.  In the sorted deposit, too,
- * particles that the reference stencil treats as out of range (base index outside the mesh, or two
- * coordinates left of it) are added to a mesh with global atomics.  stats (nullable) receives the
- * deposited mass (PK_STATS_LEN doubles).
+ * particles that the reference stencil treats as out of range (base index outside the mesh) are
+ * added to a mesh with global atomics.  stats (nullable) receives the deposited mass (PK_STATS_LEN
+ * doubles).
  * Index/fraction arithmetic follows the reference in float32: inv = 1 / ((float)box /
  * (float)n), pos = (x - xmin) * inv.
  */
