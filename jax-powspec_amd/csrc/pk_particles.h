@@ -463,15 +463,11 @@ __device__ __forceinline__ float4 bucket_record(const TileBuckets& B, const void
   return load_record_stream(sorted, (size_t)B.base[b] + (i - B.pre[b]), has_w);
 }
 
-// Half or more of the largest corner weight of a particle, at most 8.  Corner weights are <= 1, but
-// the reference stencil's truncation towards zero leaves 1 - dd in (1, 2) at a negative coordinate:
-// up to 2, 4 or 8 with one, two or three of them.  (One fits the conversion below as it is.  The count
-// tests it: a conversion in 64 bits for such records in the mesh deposit took 1% of a call at 512^3.)
-template <int ST = -1>
-__device__ __forceinline__ float corner_weight_bound(const ScatterArgs& a, float px, float py, float pz) {
-  const int stencil = ST >= 0 ? ST : a.stencil;
-  return stencil == PK_STENCIL_CIC_REF && __builtin_amdgcn_fmed3f(px, py, pz) < 0.0f ? 8.0f : 1.0f;
-}
+// Half or more of the largest corner weight of the reference stencil's particles, from the least of their
+// middle coordinates.  Weights are <= 1, but truncation towards zero leaves 1 - dd in (1, 2) at a negative
+// coordinate: up to 2, 4 or 8 with one, two or three of them.  (One fits the conversion below as it
+// is.  The count finds them: a conversion in 64 bits in the mesh deposit took 1% of a call at 512^3.)
+__device__ __forceinline__ float corner_weight_bound(float middle) { return middle < 0.0f ? 8.0f : 1.0f; }
 
 // 64-bit fixed-point deposit value (two's complement) of a weight already multiplied by
 // the scale S = 2^(30 - e) with 2^e > max |w| corner_weight_bound: |v| < 2^30, or 2^31 at one negative

@@ -84,7 +84,7 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
   const int64_t lo = (int64_t)bx * g.chunk;
   const int64_t hi = min(lo + (int64_t)g.chunk, a.np);
   double ws = 0.0;
-  float wm = 0.0f;
+  float wm = 0.0f, mid = 0.0f;   // mid: the least middle coordinate, if negative
   // CNT_UNROLL particles per thread and iteration: their loads are all in flight before
   // the first key is computed
   for (int64_t i0 = lo + tid; i0 < hi; i0 += (int64_t)CNT_NT * CNT_UNROLL) {
@@ -103,10 +103,12 @@ __device__ __forceinline__ void bucket_count_body(const Job& j, int bx, CountSha
         if (packed) atomicAdd(&hist[key >> 1], 1u << (16 * (key & 1)));
         else atomicAdd(&hist[key], 1u);
         ws += (double)w[u];
-        wm = fmaxf(wm, fabsf(w[u]) * corner_weight_bound<ST>(a, px[u], py[u], pz[u]));
+        wm = fmaxf(wm, fabsf(w[u]));
+        if ((ST >= 0 ? ST : a.stencil) == PK_STENCIL_CIC_REF) mid = fminf(mid, __builtin_amdgcn_fmed3f(px[u], py[u], pz[u]));
       }
     }
   }
+  wm *= corner_weight_bound(mid);
   atomicMax(&wmax_bits, __float_as_uint(wm));   // non-negative floats order like their bits
   __syncthreads();
   if (tid == 0) j.wmax[bx] = (double)__uint_as_float(wmax_bits);
@@ -215,8 +217,8 @@ __device__ __forceinline__ void weight_stats_body(const Job& j) {
   if (threadIdx.x == 0) {
     const double n = (double)j.a.n;
     j.stats[3] = t / (n * n * n);
-    // fixed-point scale S = 2^30 / 2^e, max |w| times the particle's corner_weight_bound < 2^e: every
-    // deposit |rint(w W S)| < 2^31, so it converts through int32
+    // fixed-point scale S = 2^30 / 2^e, max |w| corner_weight_bound < 2^e: every deposit
+    // |rint(w W S)| < 2^31, so it converts through int32
     int e = 0;
     const double wmax = __longlong_as_double((long long)wmax_bits);
     if (wmax > 0.0 && wmax < 1e300) (void)frexp(wmax, &e);
